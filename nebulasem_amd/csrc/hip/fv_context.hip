@@ -68,7 +68,8 @@ struct nsem_fv {
     uint64_t nghost = 0;
     FvDivInput div{};
     // CG work
-    Buf x, r, z, p, Ap, x32, r32, z32, p32, Ap32, e32, b32, y64, slots, sc, tmp;
+    Buf x, r, z, p, Ap, x32, r32, z32, p32, Ap32, e32, b32, y64, slots, sc, tmp, posts, faces;
+    FvBoxes boxes64, boxes32;            // the on-chip conjugate gradient's work-groups
     std::vector<int32_t> patch_kind;
     ~nsem_fv() {
         if (ev0) (void)hipEventDestroy(ev0);
@@ -325,6 +326,17 @@ static int fv_build(nsem_fv& dref, const Geometry& g, size_t npatch, const std::
     HIP_TRY(d->slots.alloc(kCgSlots * 4 * sizeof(double)));
     HIP_TRY(d->sc.alloc(sizeof(CgScalars)));
     HIP_TRY(d->tmp.alloc(8 * sizeof(double)));
+    HIP_TRY(d->posts.alloc(kFvSlotWords * sizeof(uint64_t)));
+    {
+        int dev = 0, coop = 0, cus = 0;
+        HIP_TRY(hipGetDevice(&dev));
+        HIP_TRY(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+        HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        d->boxes64 = fv_resident_boxes(A, coop ? cus : 1);
+        d->boxes32 = fv_resident_boxes(B, coop ? cus : 1);
+        HIP_TRY(d->faces.alloc(std::max((size_t)d->boxes64.groups * d->boxes64.face_cells * sizeof(double),
+                                        (size_t)d->boxes32.groups * d->boxes32.face_cells * sizeof(float))));
+    }
     HIP_TRY(hipMemcpyAsync(d->su.p, subc.data(), n * sizeof(double), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));
     return NSEM_OK;
@@ -427,7 +439,7 @@ int nsem_fv_apply(nsem_fv* d, const double* x, double* y) {
 namespace {
 
 template <typename R>
-int run_cg(nsem_fv* d, const FvOp<R>& A, const R* b, R* x, R* r, R* z, R* p, R* Ap, int mode, double tol,
+int run_cg(nsem_fv* d, const FvOp<R>& A, const FvBoxes& boxes, const R* b, R* x, R* r, R* z, R* p, R* Ap, int mode, double tol,
            int max_it, CgScalars& hs) {
     hipStream_t s = d->stream;
     CgScalars* sc = d->sc.as<CgScalars>();
@@ -438,6 +450,17 @@ int run_cg(nsem_fv* d, const FvOp<R>& A, const R* b, R* x, R* r, R* z, R* p, R* 
     init.keep_going = (mode & NSEM_FV_KEEP_GOING) ? 1 : 0;
     HIP_TRY(hipMemcpyAsync(sc, &init, sizeof(init), hipMemcpyHostToDevice, s));
     HIP_TRY(fv_cg_init<R>(A, b, x, r, z, p, sc, d->slots.as<double>(), s));
+    // on the chip where the system fits: 4096 iterations a launch (some 50 ms
+    // at most), then the host looks and the next launch carries on
+    if (boxes.groups) {
+        while (true) {
+            HIP_TRY(fv_cg_resident<R>(A, boxes, 4096, x, r, d->faces.as<R>(), p, sc, d->posts.as<uint64_t>(), s));
+            HIP_TRY(hipMemcpyAsync(&hs, sc, sizeof(hs), hipMemcpyDeviceToHost, s));
+            HIP_TRY(hipStreamSynchronize(s));
+            if (hs.aborted) return nsem_fail(NSEM_EDEVICE, "a work-group of the conjugate gradient never arrived");
+            if (hs.done) return NSEM_OK;
+        }
+    }
     int launched = 0;
     int batch = 8;
     while (true) {
@@ -468,7 +491,7 @@ extern "C" int nsem_fv_solve(nsem_fv* d, double* x_io, int32_t mode, double tol,
     CgScalars hs{};
     int rc = NSEM_OK;
     if (mode <= 1) {
-        rc = run_cg<double>(d, d->A64, d->su.as<double>(), d->x.as<double>(), d->r.as<double>(), d->z.as<double>(),
+        rc = run_cg<double>(d, d->A64, d->boxes64, d->su.as<double>(), d->x.as<double>(), d->r.as<double>(), d->z.as<double>(),
                             d->p.as<double>(), d->Ap.as<double>(), mode | keep_going, tol, max_it, hs);
         if (rc) return rc;
         res->iterations = hs.iters;
@@ -496,7 +519,7 @@ extern "C" int nsem_fv_solve(nsem_fv* d, double* x_io, int32_t mode, double tol,
             if (rel <= tol || total >= max_it) break;
             HIP_TRY(hipMemsetAsync(d->e32.p, 0, n * sizeof(float), s));
             const double inner_tol = std::max(1e-5, 0.5 * tol / std::max(rel, 1e-300));
-            rc = run_cg<float>(d, d->A32, d->b32.as<float>(), d->e32.as<float>(), d->r32.as<float>(),
+            rc = run_cg<float>(d, d->A32, d->boxes32, d->b32.as<float>(), d->e32.as<float>(), d->r32.as<float>(),
                                d->z32.as<float>(), d->p32.as<float>(), d->Ap32.as<float>(), 1,
                                std::min(inner_tol, 1e-2), max_it - total, hs);
             if (rc) return rc;

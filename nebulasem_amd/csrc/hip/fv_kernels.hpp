@@ -30,7 +30,31 @@ struct CgScalars {
     double res_ref, res0_ref, res_true, rnorm0, tol;
     int32_t iters, max_it, done, breakdown, mode;  // mode 0: reference criterion, 1: |r|/|b|
     int32_t keep_going;  // 1: a non-positive p.Ap does not stop the iteration (the reference's loop)
+    int32_t aborted;     // 1: an on-chip launch gave up waiting for one of its work-groups
 };
+
+// Sum over the 64 lanes, valid in lane 63, by DPP moves: shifts within the
+// rows of 16 lanes, then the row broadcasts.  (The shuffle form goes through
+// LDS six times: some 120 cycles a step against 20.)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+// Sum over each row of 16 lanes, valid in its last lane.
+__device__ __forceinline__ double row_sum(double v) {
+    v = dpp_add<0x111, 0xf>(v);   // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    return dpp_add<0x118, 0xf>(v);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v = row_sum(v);
+    v = dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+}
+__device__ __forceinline__ double sdiv(double p, double q) { return q != 0 ? p / q : 0; }
 
 struct FvDivInput {
     uint64_t ncells;
@@ -52,6 +76,24 @@ hipError_t fv_cg_init(const FvOp<R>& A, const R* b, const R* x, R* r, R* z, R* p
 template <typename R>
 hipError_t fv_cg_iterations(const FvOp<R>& A, int count, R* x, R* r, R* z, R* p, R* Ap, CgScalars* sc,
                             double* slots, hipStream_t s);
+// The on-chip form of the iteration (fv_resident.hip): the grid in boxes of
+// bx x by x bz cells, gx x gy x gz of them, one per work-group; groups = 0:
+// the system does not fit.
+struct FvBoxes {
+    uint32_t bx = 0, by = 0, bz = 0, gx = 0, gy = 0, gz = 0, groups = 0;
+    uint32_t face_cells = 0;   // values of a group in the face buffer
+    size_t lds = 0;
+};
+constexpr int kFvMaxGroups = 256;
+constexpr int kFvSlotWords = 2 * 4 * kFvMaxGroups + 3 * 256;
+// max_groups: the work-groups that can be resident together (one per CU).
+template <typename R>
+FvBoxes fv_resident_boxes(const FvOp<R>& A, int max_groups);
+// At most `rounds` iterations.  faces: groups * face_cells values; slots:
+// kFvSlotWords words.
+template <typename R>
+hipError_t fv_cg_resident(const FvOp<R>& A, const FvBoxes& g, int rounds, R* x, R* r, R* faces, R* p, CgScalars* sc,
+                          uint64_t* slots, hipStream_t s);
 template <typename R>
 hipError_t fv_norm2(uint64_t n, const R* v, double* out, double* slots, hipStream_t s);
 hipError_t fv_residual64(const FvOp<double>& A, const double* b, const double* x, double* y, float* y32,

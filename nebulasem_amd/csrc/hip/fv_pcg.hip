@@ -34,12 +34,6 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kMarch = 4;   // x-planes per pass of the structured SpMV march
 
-template <typename R>
-__device__ __forceinline__ R wave_sum(R v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;
-}
-
 // Block sum of NV values into slots[blockIdx.x*NV + j].
 template <int NV>
 __device__ void block_partials(double (&v)[NV], double* slots) {
@@ -47,7 +41,7 @@ __device__ void block_partials(double (&v)[NV], double* slots) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     for (int j = 0; j < NV; j++) {
         double s = wave_sum(v[j]);
-        if (lane == 0) red[wid][j] = s;
+        if (lane == 63) red[wid][j] = s;
     }
     __syncthreads();
     if (threadIdx.x == 0)
@@ -75,8 +69,6 @@ __device__ void reduce_slots(const double* slots, unsigned nblocks, double (&out
     }
     for (int j = 0; j < NV; j++) out[j] = red[0][j];
 }
-
-__device__ __forceinline__ double sdiv(double p, double q) { return q != 0 ? p / q : 0; }
 
 template <typename R>
 __device__ __forceinline__ R apply_row(const FvOp<R>& A, const R* __restrict__ x, uint64_t n) {

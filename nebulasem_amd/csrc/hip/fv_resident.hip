@@ -1,0 +1,564 @@
+// Conjugate gradients held on the chip: one cooperative launch runs many
+// iterations with x, r and p in LDS and registers, for structured systems
+// small enough that 256 CUs hold them (16 cells a thread, 2.1 M cells).
+//
+// The streaming iteration of fv_pcg.hip is five dependent launches, each of
+// which reads and writes whole vectors; below a few million cells the
+// launches and their drains are most of its time.  Here the grid is cut into
+// boxes, one per work-group, and an iteration is two exchanges of all
+// work-groups:
+//
+//   A: Ap = A p from LDS (the box and one layer of halo); the partials of
+//      p.Ap are posted; every group sums the posts of all groups: alpha
+//   B: x += alpha p, r -= alpha Ap, z = r / ap; z of the box's faces is
+//      written to memory and the partials of r.z, z.z, x.x, r.r are posted;
+//      every group sums them: beta, residuals, stop.  p = z + beta p is then
+//      formed for the own cells and again for the halo, from the neighbours'
+//      face z, so p itself is never exchanged and no third exchange is
+//      needed.
+//
+// An exchange: every group posts its sums, one 8-byte store per value into its
+// own slot; group 0 polls the slots, adds them in a fixed order and writes the
+// totals kCopies times, and every group polls a copy.  (All groups polling all
+// slots is one hop less, but 256 pollers of the same lines wait some 3 us for
+// each other; so it is about 1.2 us.)  A word not yet written holds kEmpty (a
+// NaN pattern that no sum is allowed to have).  Sets of slots and of copies
+// rotate by the number s of the exchange: a group that has the totals of s
+// knows that its slot of s has been read and empties it, visibly before its
+// post of s + 1, hence before group 0 polls that set again at s + 2; group 0,
+// having all posts of s, knows that all have read the totals of s - 1 and
+// empties those, visibly before it writes the totals of s + 1, hence before
+// anyone polls that set again at s + 2.  Face z, posts, totals and the
+// emptying are agent-scope accesses, which write through to and read from the
+// level that all XCDs share; every wave waits for its z stores before the
+// group's barrier and the posting wave for its own stores before the post, so
+// a post is never seen before what it stands for, and no L2 is written back or
+// invalidated (with release and acquire fences at agent scope an iteration
+// took 135 us at 128^3).  A face buffer may be written again in the next B:
+// the neighbour has read it before its post of the A between.  The launch is
+// cooperative, so all groups are resident; a poll gives up after kPollLimit
+// rounds all the same, and the launch then ends with CgScalars::aborted set.
+//
+// The row, update and scalar arithmetic is that of fv_pcg.hip operation for
+// operation (a missing neighbour is a halo cell whose p stays 0); only the
+// order in which the partial sums are added differs (it is fixed, so runs
+// repeat bit for bit).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "fv_kernels.hpp"
+
+namespace nsem {
+
+namespace {
+
+// 8 waves, 2 per SIMD, so a lane may hold 256 VGPRs of cells (16 waves of 128
+// hold less: what is not a cell takes some 40 registers of either)
+constexpr int kT = 512;
+constexpr int kWaves = kT / 64;
+constexpr int kMaxGroups = kFvMaxGroups;         // 4 per lane of a wave
+constexpr int kTasks = 5;                        // face cells per thread at most
+constexpr size_t kHoldCouplings = 48;             // bytes a lane and array: 6 cells FP64, 12 FP32
+constexpr uint32_t kNone = ~0u;
+constexpr uint64_t kEmpty = ~0ull;
+constexpr uint32_t kPollLimit = 1u << 21;
+constexpr size_t kLdsLimit = 160 * 1024 - 2048;  // the rest: static scratch
+
+template <typename R>
+__device__ __forceinline__ void put(R* p, R v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T get(const T* p) {
+    return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Wait until this wave's stores have been performed.
+__device__ __forceinline__ void drain() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+}
+
+constexpr int kCopies = 16;
+constexpr int kCopyWords = 16;                   // 128 bytes apart
+// words: two sets of posts [4][kMaxGroups], three of totals [kCopies][kCopyWords]
+constexpr int kPosts = 4 * kMaxGroups, kTotals = kCopies * kCopyWords;
+static_assert(2 * kPosts + 3 * kTotals == kFvSlotWords, "slot words");
+
+struct Scratch {
+    double red[4][kWaves];
+    double tot[4];
+    int dead;
+};
+
+// This wave's share of NV sums, for exchange() after a barrier.
+template <int NV>
+__device__ __forceinline__ void reduce_wave(const double (&v)[NV], Scratch& sh) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const double s = wave_sum(v[j]);
+        if (lane == 63) sh.red[j][wid] = s;
+    }
+}
+
+// wave_sum on every lane.
+__device__ __forceinline__ double wave_total(double v) {
+    v = wave_sum(v);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// Poll one word until it is written; kEmpty when it never is.
+__device__ __forceinline__ uint64_t wait_word(const uint64_t* w) {
+    uint64_t bits = get(w);
+    for (uint32_t tries = 0; bits == kEmpty && tries < kPollLimit; tries++) bits = get(w);
+    return bits;
+}
+__device__ __forceinline__ uint64_t word_of(double v) {
+    const uint64_t bits = __double_as_longlong(v);
+    return bits == kEmpty ? 0x7ff8000000000000ull : bits;
+}
+
+// Sums of the NV values of reduce_wave over all threads of all work-groups,
+// the same on every thread of every group.  True when a group never posted.
+template <int NV, bool ONE>
+__device__ __forceinline__ bool exchange(double (&v)[NV], uint32_t groups, uint64_t* words, uint32_t& seq, Scratch& sh) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (wid == 0) {
+        // row j of the wave sums value j over the waves: valid in lane 16 j + 15
+        double s = row_sum(lane < 16 * NV && (lane & 15) < kWaves ? sh.red[lane >> 4][lane & 15] : 0.0);
+        if constexpr (ONE) {
+            if ((lane & 15) == 15 && lane < 16 * NV) sh.tot[lane >> 4] = s;
+        } else {
+            uint64_t* posts = words + (seq & 1) * kPosts;
+            uint64_t* totals = words + 2 * kPosts + (seq % 3) * kTotals;
+            drain();
+            if ((lane & 15) == 15 && lane < 16 * NV) put(posts + (lane >> 4) * kMaxGroups + blockIdx.x, word_of(s));
+            bool dead = false;
+            if (blockIdx.x == 0) {
+                // lane l sums the posts of groups l, l + 64, ...; all words are
+                // read together, and again until none is empty
+                constexpr int kC = kMaxGroups / 64;
+                uint64_t bits[NV][kC];
+                uint32_t tries = 0;
+                do {
+                    dead = false;
+#pragma unroll
+                    for (int j = 0; j < NV; j++)
+#pragma unroll
+                        for (int c = 0; c < kC; c++)
+                            bits[j][c] = c * 64 + lane < (int)groups ? get(posts + j * kMaxGroups + c * 64 + lane) : 0;
+#pragma unroll
+                    for (int j = 0; j < NV; j++)
+#pragma unroll
+                        for (int c = 0; c < kC; c++) dead = dead || bits[j][c] == kEmpty;
+                } while (dead && ++tries < kPollLimit);
+                double got[NV];
+#pragma unroll
+                for (int j = 0; j < NV; j++)
+                    got[j] = (__longlong_as_double(bits[j][0]) + __longlong_as_double(bits[j][1])) +
+                             (__longlong_as_double(bits[j][2]) + __longlong_as_double(bits[j][3]));
+                // the totals of the exchange before have been read by all
+                put(words + 2 * kPosts + ((seq + 2) % 3) * kTotals + (lane >> 2) * kCopyWords + (lane & 3), kEmpty);
+                double mine = 0;
+#pragma unroll
+                for (int j = 0; j < NV; j++) {
+                    const double t = wave_total(got[j]);
+                    if ((lane & 3) == j) mine = t;
+                }
+                if (!__any(dead) && (lane & 3) < NV)
+                    put(totals + (lane >> 2) * kCopyWords + (lane & 3), word_of(mine));
+                if (lane < NV) sh.tot[lane] = mine;
+            } else if (lane < NV) {
+                const uint64_t bits = wait_word(totals + (blockIdx.x % kCopies) * kCopyWords + lane);
+                dead = bits == kEmpty;
+                sh.tot[lane] = __longlong_as_double(bits);
+            }
+            if (__any(dead) && lane == 0) sh.dead = 1;
+            // group 0 has read this group's posts: empty them
+            if (lane < 4) put(posts + lane * kMaxGroups + blockIdx.x, kEmpty);
+        }
+    }
+    seq++;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NV; j++) v[j] = sh.tot[j];
+    return !ONE && sh.dead;
+}
+
+// Byte offset access from a scalar base.
+template <typename T>
+__device__ __forceinline__ T at(const T* base, uint32_t off) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off);
+}
+
+// The six couplings (x+ x- y+ y- z+ z-) of the cell at byte offset o; sx, sy:
+// byte strides of x and y.  (Below the first cell the halo's p is 0 and any will do.)
+template <typename R>
+__device__ __forceinline__ void couplings(const FvOp<R>& A, uint32_t o, uint32_t sx, uint32_t sy, R (&c)[6]) {
+    const R *c0 = A.cpl, *c1 = A.cpl + A.n, *c2 = A.cpl + 2 * A.n;
+    c[0] = at(c0, o);
+    c[1] = at(c0, o >= sx ? o - sx : 0);
+    c[2] = at(c1, o);
+    c[3] = at(c1, o >= sy ? o - sy : 0);
+    c[4] = at(c2, o);
+    c[5] = at(c2, o >= (uint32_t)sizeof(R) ? o - (uint32_t)sizeof(R) : 0);
+}
+
+// K cells per thread; UNI: the couplings are the three constants A.cu; ONE:
+// a single work-group, nothing to exchange.
+template <typename R, int K, bool UNI, bool ONE>
+__global__ void __launch_bounds__(kT) cg_resident_kernel(FvOp<R> A, FvBoxes g, R* __restrict__ x, R* __restrict__ r,
+                                                         R* faces, R* __restrict__ p, CgScalars* sc, uint64_t* slots,
+                                                         int max_rounds) {
+    if (sc->done) return;
+    // diag and 1/diag stay in registers where both fit beside the vectors
+    // (HOLD), else one array holds them in turn, each read again while an
+    // exchange is waited for; couplings stay (HOLDC), or are read one cell
+    // ahead of their use (from L2)
+    constexpr bool HOLD = K * sizeof(R) <= 64, HOLDC = !UNI && K * sizeof(R) <= kHoldCouplings;
+    constexpr int KH = HOLD ? K : 1, KC = HOLDC ? K : 1, KO = HOLD && (UNI || HOLDC) ? 1 : K;
+    constexpr uint32_t S = sizeof(R);
+    extern __shared__ unsigned char lds_cg[];
+    __shared__ Scratch sh;
+    const uint32_t sj = g.bz + 2, si = (g.by + 2) * sj;   // strides of the box with its halo
+    const uint32_t box = g.bx * g.by * g.bz, plane = g.by * g.bz;
+    R* P = reinterpret_cast<R*>(lds_cg);
+    R* Z = P + (g.bx + 2) * si;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t gk = blockIdx.x % g.gz, gj = (blockIdx.x / g.gz) % g.gy, gi = blockIdx.x / (g.gz * g.gy);
+    const uint32_t i0 = gi * g.bx, j0 = gj * g.by, k0 = gk * g.bz;
+    const uint32_t sx = (uint32_t)A.sx, nz = (uint32_t)A.nz;
+
+    if (tid == 0) sh.dead = 0;
+    for (uint32_t q = tid; q < (g.bx + 2) * si; q += kT) P[q] = R(0);
+    __syncthreads();
+    R xx[K], rr[K], ap[K], dg[K], id[KH];
+    R cxp[KC], cxm[KC], cyp[KC], cym[KC], czp[KC], czm[KC];
+    uint32_t slot[K];    // byte offset in P; the top bit: no cell
+    uint32_t off[KO];    // byte offset in the cell arrays
+#pragma unroll
+    for (int u = 0; u < K; u++) {
+        const uint32_t q = u * kT + tid;
+        const uint32_t i = q / plane, j = (q - i * plane) / g.bz, k = q - i * plane - j * g.bz;
+        const uint32_t gx = i0 + i, gy = j0 + j, gz = k0 + k;
+        const bool ok = q < box && gx < (uint32_t)A.nx && gy < (uint32_t)A.ny && gz < (uint32_t)A.nz;
+        // a place without a cell reads the box's first cell
+        const uint32_t c = ok ? gx * sx + gy * nz + gz : 0;
+        const uint32_t sl = ok ? (i + 1) * si + (j + 1) * sj + k + 1 : si + sj + 1;
+        slot[u] = sl * S | (ok ? 0u : 0x80000000u);
+        if constexpr (KO > 1) off[u] = c * S;
+        else off[0] = 0;
+        rr[u] = xx[u] = R(0);
+        dg[u] = A.diag[c];
+        if constexpr (HOLD) id[u] = A.idiag[c];
+        if constexpr (HOLDC) {
+            const R *c0 = A.cpl, *c1 = A.cpl + A.n, *c2 = A.cpl + 2 * A.n;
+            cxp[u] = c0[c]; cyp[u] = c1[c]; czp[u] = c2[c];
+            cxm[u] = gx > 0 && ok ? c0[c - sx] : R(0);
+            cym[u] = gy > 0 && ok ? c1[c - nz] : R(0);
+            czm[u] = gz > 0 && ok ? c2[c - 1] : R(0);
+        }
+        if (ok) {
+            rr[u] = r[c];
+            xx[u] = x[c];
+            P[sl] = p[c];
+        }
+    }
+    // face cells: task t = u kT + tid writes the z of one own face cell to
+    // faces[group][t] and reads the z of the halo cell beside it from the
+    // neighbour's opposite face
+    const uint32_t nfx = g.by * g.bz, nfy = g.bx * g.bz, nfz = g.bx * g.by, nf = 2 * (nfx + nfy + nfz);
+    uint32_t cell[ONE ? 1 : kTasks];   // index in Z | index of the halo cell in P << 16; kNone: no task
+    uint32_t from[ONE ? 1 : kTasks];   // byte offset in faces
+    if constexpr (!ONE) {
+#pragma unroll
+        for (int u = 0; u < kTasks; u++) {
+            const uint32_t t = u * kT + tid;
+            cell[u] = kNone;
+            from[u] = 0;
+            if (t >= nf) continue;
+            uint32_t d, l, h;      // direction, place on the face, side
+            if (t < 2 * nfx) { d = 0; h = t >= nfx; l = t - h * nfx; }
+            else if (t < 2 * (nfx + nfy)) { d = 1; l = t - 2 * nfx; h = l >= nfy; l -= h * nfy; }
+            else { d = 2; l = t - 2 * (nfx + nfy); h = l >= nfz; l -= h * nfz; }
+            const uint32_t nb = d == 2 ? g.by : g.bz, a = l / nb, b = l - a * nb;
+            // the box's extents (cut at the grid's end)
+            const uint32_t ex = min(g.bx, (uint32_t)A.nx - i0), ey = min(g.by, (uint32_t)A.ny - j0),
+                           ez = min(g.bz, (uint32_t)A.nz - k0);
+            const uint32_t i = d == 0 ? (h ? ex - 1 : 0) : a, j = d == 1 ? (h ? ey - 1 : 0) : d == 0 ? a : b,
+                           k = d == 2 ? (h ? ez - 1 : 0) : b;
+            const bool edge = d == 0 ? (h ? gi + 1 == g.gx : gi == 0)
+                                     : d == 1 ? (h ? gj + 1 == g.gy : gj == 0) : (h ? gk + 1 == g.gz : gk == 0);
+            if (edge || i >= ex || j >= ey || k >= ez) continue;
+            const uint32_t step = d == 0 ? g.gy * g.gz : d == 1 ? g.gz : 1;
+            const uint32_t nbr = h ? blockIdx.x + step : blockIdx.x - step;
+            const uint32_t nfd = d == 0 ? nfx : d == 1 ? nfy : nfz;
+            const uint32_t sd = d == 0 ? si : d == 1 ? sj : 1;
+            const uint32_t sl = (i + 1) * si + (j + 1) * sj + k + 1;
+            cell[u] = ((i * g.by + j) * g.bz + k) | (h ? sl + sd : sl - sd) << 16;
+            from[u] = (nbr * nf + (h ? t - nfd : t + nfd)) * S;
+            // p of the halo cell, from memory this once
+            const uint32_t c = (i0 + i) * sx + (j0 + j) * nz + k0 + k, st = d == 0 ? sx : d == 1 ? nz : 1;
+            P[h ? sl + sd : sl - sd] = p[h ? c + st : c - st];
+        }
+    }
+    __syncthreads();
+
+    double rz = sc->rz, alpha_d = 0, beta_d = 0, pap = sc->pAp, res_ref = sc->res_ref, res_true = sc->res_true;
+    const double tol = sc->tol, bnorm = sc->bnorm;
+    const int max_it = sc->max_it, mode = sc->mode, keep_going = sc->keep_going;
+    int iters = sc->iters, breakdown = sc->breakdown, done = 0;
+    bool dead = false;
+    uint32_t seq = 0;
+    const char* Pb = reinterpret_cast<const char*>(P);
+
+    for (int round = 0; round < max_rounds && !done && !dead; round++) {
+        // opaque here, so that no address of an unrolled cell is kept in
+        // registers over the iterations
+#pragma unroll
+        for (int u = 0; u < K; u++) __asm__ volatile("" : "+v"(slot[u]));
+        if constexpr (!ONE) {
+#pragma unroll
+            for (int u = 0; u < kTasks; u++) __asm__ volatile("" : "+v"(cell[u]), "+v"(from[u]));
+        }
+        if constexpr (KO > 1) {
+#pragma unroll
+            for (int u = 0; u < K; u++) __asm__ volatile("" : "+v"(off[u]));
+        }
+        double va[1] = {0};
+        R cn[6];
+        if constexpr (!UNI && !HOLDC) couplings(A, off[0], sx * S, nz * S, cn);
+#pragma unroll
+        for (int u = 0; u < K; u++) {
+            const R* q = reinterpret_cast<const R*>(Pb + (slot[u] & 0x7fffffffu));
+            const R pc = q[0], pxp = q[si], pxm = *(q - si), pyp = q[sj], pym = *(q - sj), pzp = q[1], pzm = *(q - 1);
+            R k0, k1, k2, k3, k4, k5;
+            if constexpr (UNI) {
+                k0 = k1 = A.cu[0]; k2 = k3 = A.cu[1]; k4 = k5 = A.cu[2];
+            } else if constexpr (HOLDC) {
+                k0 = cxp[u]; k1 = cxm[u]; k2 = cyp[u]; k3 = cym[u]; k4 = czp[u]; k5 = czm[u];
+            } else {
+                k0 = cn[0]; k1 = cn[1]; k2 = cn[2]; k3 = cn[3]; k4 = cn[4]; k5 = cn[5];
+                if (u + 1 < K) couplings(A, off[u + 1 < K ? u + 1 : u], sx * S, nz * S, cn);
+            }
+            R acc = pc * dg[u];
+            acc -= pxp * k0;
+            acc -= pxm * k1;
+            acc -= pyp * k2;
+            acc -= pym * k3;
+            acc -= pzp * k4;
+            acc -= pzm * k5;
+            ap[u] = acc;
+            if (!(slot[u] >> 31)) va[0] += (double)pc * (double)acc;
+            // (the scheduler would otherwise raise every cell's reads to the
+            // front and spill)
+            if (K > 4 && u % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (!HOLD) {
+#pragma unroll
+            for (int u = 0; u < K; u++) dg[u] = at(A.idiag, off[u]);
+        }
+        reduce_wave<1>(va, sh);
+        __syncthreads();
+        dead = exchange<1, ONE>(va, g.groups, slots, seq, sh);
+        if (dead) break;
+        pap = va[0];
+        alpha_d = sdiv(rz, pap);
+        if (!(pap > 0) && rz != 0 && !keep_going) breakdown = 1;
+        const R alpha = (R)alpha_d;
+        double vb[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int u = 0; u < K; u++) {
+            const R i_d = HOLD ? id[HOLD ? u : 0] : dg[u];
+            const R xn = xx[u] + *reinterpret_cast<const R*>(Pb + (slot[u] & 0x7fffffffu)) * alpha;
+            const R rn = rr[u] + ap[u] * (-alpha);
+            const R zn = rn * i_d;
+            if (!(slot[u] >> 31)) {
+                xx[u] = xn;
+                rr[u] = rn;
+                Z[u * kT + tid] = zn;
+                vb[0] += (double)rn * (double)zn;
+                vb[1] += (double)zn * (double)zn;
+                vb[2] += (double)xn * (double)xn;
+                vb[3] += (double)rn * (double)rn;
+            }
+            if (K > 4 && u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (!HOLD) {
+#pragma unroll
+            for (int u = 0; u < K; u++) dg[u] = at(A.diag, off[u]);
+        }
+        reduce_wave<4>(vb, sh);
+        __syncthreads();
+        if constexpr (!ONE) {
+            R* mine = faces + (size_t)blockIdx.x * nf + tid;
+#pragma unroll
+            for (int u = 0; u < kTasks; u++)
+                if (cell[u] != kNone) put(mine + u * kT, Z[cell[u] & 0xffffu]);
+            drain();
+            __syncthreads();
+        }
+        dead = exchange<4, ONE>(vb, g.groups, slots, seq, sh);
+        if (dead) break;
+        R fz[ONE ? 1 : kTasks];
+        if constexpr (!ONE) {
+#pragma unroll
+            for (int u = 0; u < kTasks; u++)
+                fz[u] = get(reinterpret_cast<const R*>(reinterpret_cast<const char*>(faces) + from[u]));
+        }
+        beta_d = sdiv(vb[0], rz);
+        rz = vb[0];
+        iters++;
+        res_ref = sqrt(sdiv(fabs(vb[1]), fabs(vb[2])));
+        res_true = bnorm > 0 ? sqrt(vb[3]) / bnorm : 0;
+        const double crit = mode == 0 ? res_ref : res_true;
+        if (crit <= tol || iters >= max_it || breakdown) { done = 1; break; }
+        const R beta = (R)beta_d;
+#pragma unroll
+        for (int u = 0; u < K; u++) {
+            R* q = reinterpret_cast<R*>(lds_cg + (slot[u] & 0x7fffffffu));
+            if (!(slot[u] >> 31)) *q = Z[u * kT + tid] + *q * beta;
+            if (K > 4 && u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (!ONE) {
+#pragma unroll
+            for (int u = 0; u < kTasks; u++) {
+                R* q = P + (cell[u] >> 16);
+                if (cell[u] != kNone) *q = fz[u] + *q * beta;
+            }
+        }
+        __syncthreads();
+    }
+    // x, r, p back to memory: the next launch carries on from them
+#pragma unroll
+    for (int u = 0; u < K; u++) {
+        if (slot[u] >> 31) continue;
+        const uint32_t q = u * kT + tid;
+        const uint32_t i = q / plane, j = (q - i * plane) / g.bz, k = q - i * plane - j * g.bz;
+        const uint32_t c = (i0 + i) * sx + (j0 + j) * nz + k0 + k;
+        x[c] = xx[u];
+        r[c] = rr[u];
+        p[c] = *reinterpret_cast<const R*>(Pb + slot[u]);
+    }
+    if (blockIdx.x == 0 && tid == 0) {
+        sc->pAp = pap;
+        sc->alpha = alpha_d;
+        sc->beta = beta_d;
+        sc->rz = rz;
+        sc->iters = iters;
+        sc->res_ref = res_ref;
+        sc->res_true = res_true;
+        sc->breakdown = breakdown;
+        sc->done = done;
+    }
+    if (dead && tid == 0) sc->aborted = 1;
+}
+
+__global__ void __launch_bounds__(256) clear_slots_kernel(uint64_t* slots) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < (uint32_t)kFvSlotWords) slots[i] = kEmpty;
+}
+
+template <typename R, int K, bool UNI, bool ONE>
+hipError_t launch(const FvOp<R>& A, const FvBoxes& g, R* x, R* r, R* faces, R* p, CgScalars* sc, uint64_t* slots,
+                  int rounds, hipStream_t s) {
+    auto kernel = cg_resident_kernel<R, K, UNI, ONE>;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds);
+    if (e != hipSuccess) return e;
+    if constexpr (ONE) {
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(kT), g.lds, s, A, g, x, r, faces, p, sc, slots, rounds);
+        return hipGetLastError();
+    } else {
+        FvOp<R> a = A;
+        FvBoxes gr = g;
+        void* args[] = {&a, &gr, &x, &r, &faces, &p, &sc, &slots, &rounds};
+        hipLaunchKernelGGL(clear_slots_kernel, dim3((kFvSlotWords + 255) / 256), dim3(256), 0, s, slots);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(kernel), dim3(g.groups), dim3(kT), args,
+                                          (unsigned)g.lds, s);
+    }
+}
+
+// The instantiated cells per thread.
+uint32_t rounded(uint32_t k) {
+    for (uint32_t have : {1u, 2u, 4u, 6u, 8u, 12u})
+        if (k <= have) return have;
+    return 16;
+}
+
+template <typename R, int K>
+hipError_t launch_k(const FvOp<R>& A, const FvBoxes& g, R* x, R* r, R* faces, R* p, CgScalars* sc, uint64_t* slots,
+                    int rounds, hipStream_t s) {
+    if (A.uniform)
+        return g.groups == 1 ? launch<R, K, true, true>(A, g, x, r, faces, p, sc, slots, rounds, s)
+                             : launch<R, K, true, false>(A, g, x, r, faces, p, sc, slots, rounds, s);
+    return g.groups == 1 ? launch<R, K, false, true>(A, g, x, r, faces, p, sc, slots, rounds, s)
+                         : launch<R, K, false, false>(A, g, x, r, faces, p, sc, slots, rounds, s);
+}
+
+}  // namespace
+
+// The grid's cut into boxes.  More groups mean fewer cells a thread; the
+// exchange hardly grows with them (128 x 128 x 128 FP64: 256 groups, 13.3 us an
+// iteration against 54 for the streaming kernels; 83 x 71 x 97 FP32 7.8
+// against 29; 24 x 20 x 16 5.5 against 22), so only systems of up to some
+// 4,000 cells stay in one group (12 x 12 x 12: 2.4 us).
+template <typename R>
+FvBoxes fv_resident_boxes(const FvOp<R>& A, int max_groups) {
+    FvBoxes best{};
+    if (!A.structured || A.n == 0 || A.n > (1ull << 28)) return best;
+    const uint32_t nx = A.nx, ny = A.ny, nz = A.nz;
+    const uint32_t most = (uint32_t)std::min(max_groups, kMaxGroups), max_k = 16;
+    double cost = 1e30;
+    for (uint32_t gx = 1; gx <= most && gx <= nx; gx++)
+        for (uint32_t gy = 1; gx * gy <= most && gy <= ny; gy++)
+            for (uint32_t gz = 1; gx * gy * gz <= most && gz <= nz; gz++) {
+                FvBoxes b{};
+                b.bx = (nx + gx - 1) / gx; b.by = (ny + gy - 1) / gy; b.bz = (nz + gz - 1) / gz;
+                b.gx = (nx + b.bx - 1) / b.bx; b.gy = (ny + b.by - 1) / b.by; b.gz = (nz + b.bz - 1) / b.bz;
+                b.groups = b.gx * b.gy * b.gz;
+                const uint64_t cells = (uint64_t)b.bx * b.by * b.bz;
+                const uint64_t nf = 2 * ((uint64_t)b.by * b.bz + (uint64_t)b.bx * b.bz + (uint64_t)b.bx * b.by);
+                if (cells > (uint64_t)max_k * kT || (b.groups > 1 && nf > (uint64_t)kTasks * kT)) continue;
+                b.face_cells = (uint32_t)nf;
+                b.lds = ((size_t)(b.bx + 2) * (b.by + 2) * (b.bz + 2) + ((cells + kT - 1) / kT) * kT) * sizeof(R);
+                if (b.lds > kLdsLimit) continue;
+                // cycles of an iteration, fitted to measurements: 750 a cell
+                // of a thread with all its operands held, 1700 where the
+                // couplings are read again; two exchanges 10,000 and a little
+                // for each group; one group needs no exchange
+                const uint32_t k = rounded((uint32_t)((cells + kT - 1) / kT));
+                double c = k * (!A.uniform && k * sizeof(R) > kHoldCouplings ? 1700.0 : 750.0);
+                if (b.groups > 1) c += 10000.0 + 6.0 * b.groups + 150.0 * ((nf + kT - 1) / kT);
+                if (c < cost) { cost = c; best = b; }
+            }
+    return best;
+}
+
+template <typename R>
+hipError_t fv_cg_resident(const FvOp<R>& A, const FvBoxes& g, int rounds, R* x, R* r, R* faces, R* p, CgScalars* sc,
+                          uint64_t* slots, hipStream_t s) {
+    if (g.groups == 0) return hipErrorInvalidValue;
+    switch (rounded((g.bx * g.by * g.bz + kT - 1) / kT)) {
+        case 1: return launch_k<R, 1>(A, g, x, r, faces, p, sc, slots, rounds, s);
+        case 2: return launch_k<R, 2>(A, g, x, r, faces, p, sc, slots, rounds, s);
+        case 4: return launch_k<R, 4>(A, g, x, r, faces, p, sc, slots, rounds, s);
+        case 6: return launch_k<R, 6>(A, g, x, r, faces, p, sc, slots, rounds, s);
+        case 8: return launch_k<R, 8>(A, g, x, r, faces, p, sc, slots, rounds, s);
+        case 12: return launch_k<R, 12>(A, g, x, r, faces, p, sc, slots, rounds, s);
+        default: return launch_k<R, 16>(A, g, x, r, faces, p, sc, slots, rounds, s);
+    }
+}
+
+template FvBoxes fv_resident_boxes<double>(const FvOp<double>&, int);
+template FvBoxes fv_resident_boxes<float>(const FvOp<float>&, int);
+template hipError_t fv_cg_resident<double>(const FvOp<double>&, const FvBoxes&, int, double*, double*, double*, double*,
+                                           CgScalars*, uint64_t*, hipStream_t);
+template hipError_t fv_cg_resident<float>(const FvOp<float>&, const FvBoxes&, int, float*, float*, float*, float*,
+                                          CgScalars*, uint64_t*, hipStream_t);
+
+}  // namespace nsem

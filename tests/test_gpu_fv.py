@@ -141,3 +141,32 @@ def test_fv_indefinite_operator_reports_breakdown(tmp_path):
     print(f"  rc {rc} breakdown {res.breakdown} iters {res.iterations}", flush=True)
     assert rc == 6 and res.breakdown == 1
     fv.close()
+
+
+@pytest.mark.parametrize("ndiv,mu", [((1, 1, 600), False), ((16, 16, 16), True), ((17, 16, 16), True), ((3, 5, 700), True),
+                                     ((67, 61, 59), False), ((67, 61, 59), True), ((96, 88, 80), True),
+                                     ((128, 128, 128), False)])
+def test_fv_on_chip_cg(tmp_path, ndiv, mu):
+    """The conjugate gradient held on the chip: one work-group and several,
+    boxes cut by the grid's end, one-cell-thick and long grids, held and
+    re-read couplings, and the largest system it takes.  The true residual is
+    formed by the row-per-thread apply kernel; a cell, face or halo that the
+    on-chip kernel misses shows there.  The criterion uses the recursive
+    residual, which drifts from the true one by some 1e-15 an iteration of
+    |A||x|/|b|: 1e-2 of the tolerance at most on these sizes."""
+    print(f"[gpu] fv on chip {ndiv} mu {mu}", flush=True)
+    mesh, U, p, kp, vp = potential_inputs(tmp_path, dict(name="pot_chip", ndiv=ndiv, seed=23))
+    n = mesh.info.nbcs
+    m = np.random.default_rng(29).uniform(0.5, 2.0, size=mesh.info.ncells) if mu else None
+    fv = FVPoisson(mesh, kp, vp, mu=m)
+    fv.set_rhs_divergence(U[:n], np.zeros(len(mesh.boundaries), dtype=np.int32),
+                          np.zeros((len(mesh.boundaries), 3)))
+    b = fv.rhs()
+    for mode in (1, 2):
+        x, r, rc = fv.solve(mode=mode, tol=1e-9)
+        y, r2, _ = fv.solve(mode=mode, tol=1e-9)
+        true = np.linalg.norm(b - fv.apply(x)) / np.linalg.norm(b)
+        print(f"  mode {mode} iters {r.iterations} true {true:.2e} uniform {fv.uniform}", flush=True)
+        assert rc == 0 and true <= 1.01e-9
+        assert np.array_equal(x, y) and r.iterations == r2.iterations
+    fv.close()
