@@ -184,7 +184,9 @@ int nsem_dg_rk3_tlm(nsem_dg* d, int32_t nsteps, double* dq);
  * checkpointed every `checkpoint` steps and recomputed segment by segment.
  * NSEM_ENONFINITE when the forward state or the gradient is not finite. */
 int nsem_dg_rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, double* lam);
-/* Same, returning the device time of the sweeps (forward with checkpoints,
+/* Same, the gradient to grad (lam is left as it is). */
+int nsem_dg_rk3_gradient(nsem_dg* d, int32_t nsteps, int32_t checkpoint, const double* lam, double* grad);
+/* As nsem_dg_rk3_adjoint, returning the device time of the sweeps (forward with checkpoints,
  * recomputation, backward), host transfers of lam excluded. */
 int nsem_dg_time_rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, double* lam, double* seconds);
 /* Per-step diagnostics of the current state (split or method-of-lines),
@@ -297,6 +299,8 @@ int nsem_fv_solve(nsem_fv* fv, double* x, int32_t mode, double tol, int32_t max_
  * nsem_fv_create, as Solve's applyExplicitBCs sets them), U interior cells
  * xyz, updated in place. */
 int nsem_fv_correct_velocity(nsem_fv* fv, const double* p, double* U);
+/* Same, the corrected velocity to out (U is left as it is). */
+int nsem_fv_corrected_velocity(nsem_fv* fv, const double* p, const double* U, double* out);
 
 /* ----------------------------------------------------------- measurement --
  * Device-to-device copy of `bytes` (a multiple of 16) through a plain

@@ -328,9 +328,10 @@ class DGEuler:
         return dq
 
     def rk3_adjoint(self, n, lam, checkpoint=10):
-        lam = np.array(lam, dtype=np.float64).reshape(5, -1)
-        check(lib().nsem_dg_rk3_adjoint(self._h, int(n), int(checkpoint), _pd(lam)))
-        return lam
+        lam = np.ascontiguousarray(lam, dtype=np.float64).reshape(5, -1)
+        grad = np.empty_like(lam)
+        check(lib().nsem_dg_rk3_gradient(self._h, int(n), int(checkpoint), _pd(lam), _pd(grad)))
+        return grad
 
     def time_rk3_adjoint(self, n, lam, checkpoint=10):
         """rk3_adjoint, also returning the device time of the sweeps."""
@@ -429,8 +430,10 @@ class FVPoisson:
         """U - gradf(p, true) on the interior cells (nsem_fv_correct_velocity);
         U: (n, 3), returned as a new array."""
         p = np.ascontiguousarray(p, dtype=np.float64).reshape(-1)[:self.n]
-        out = np.array(U, dtype=np.float64).reshape(-1)[:3 * self.n].copy()
-        check(lib().nsem_fv_correct_velocity(self._h, _pd(p), _pd(out)))
+        U = np.ascontiguousarray(np.asarray(U, dtype=np.float64).reshape(-1)[:3 * self.n])
+        assert p.size == self.n and U.size == 3 * self.n
+        out = np.empty_like(U)
+        check(lib().nsem_fv_corrected_velocity(self._h, _pd(p), _pd(U), _pd(out)))
         return out.reshape(-1, 3)
 
     def solve(self, x0=None, mode=0, tol=1e-10, max_it=100000, raise_on_error=True):

@@ -702,19 +702,16 @@ hipError_t workspace(nsem_dg* d, size_t n, std::vector<Field5>& out) {
     return hipSuccess;
 }
 
-hipError_t upload5(const Field5& f, const double* host, uint64_t nb, hipStream_t s) {
-    for (int v = 0; v < 5; v++) {
-        hipError_t e = hipMemcpyAsync(f.p(v), host + (size_t)v * nb, nb * sizeof(double), hipMemcpyHostToDevice, s);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+PipeColumns columns5(const Field5& f, const double* host, uint64_t nb) {
+    PipeColumns c;
+    for (int v = 0; v < 5; v++) c.add(host + (size_t)v * nb, f.p(v));
+    return c;
 }
-hipError_t download5(double* host, const Field5& f, uint64_t nb, hipStream_t s) {
-    for (int v = 0; v < 5; v++) {
-        hipError_t e = hipMemcpyAsync(host + (size_t)v * nb, f.p(v), nb * sizeof(double), hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) return e;
-    }
-    return hipStreamSynchronize(s);
+hipError_t upload5(nsem_dg* d, const Field5& f, const double* host) {
+    return d->pipe.upload(columns5(f, host, d->nb), d->nb, d->stream);
+}
+hipError_t download5(nsem_dg* d, double* host, const Field5& f, bool* finite = nullptr) {
+    return d->pipe.download(columns5(f, host, d->nb), d->nb, d->stream, finite);
 }
 hipError_t copy5(const Field5& dst, const double* const src[5], uint64_t nb, hipStream_t s) {
     for (int v = 0; v < 5; v++) {
@@ -740,14 +737,8 @@ hipError_t fwd_stage(nsem_dg* d, int stage, const double* const q[5], const doub
     a.bdt = kB[stage] * d->dev.dt;
     a.last = stage == 2;
     a.check = stage == 2;
-    a.flag = d->flag.as<int>();
+    a.flag = d->flag();
     return launch_rk_stage<double, double>(d->dev, a, d->stream);
-}
-
-bool all_finite(const double* v, uint64_t n) {
-    for (uint64_t i = 0; i < n; i++)
-        if (!std::isfinite(v[i])) return false;
-    return true;
 }
 
 struct AdjointWork {
@@ -807,14 +798,14 @@ int nsem_dg_residual_vjp(nsem_dg* d, const double* w, double* t) {
     std::vector<Field5> ws;
     HIP_TRY(workspace(d, 2, ws));
     const Field5 &W = ws[0], &T = ws[1];
-    HIP_TRY(upload5(W, w, nb, d->stream));
+    HIP_TRY(upload5(d, W, w));
     VjpArgs a{};
     for (int v = 0; v < 5; v++) {
         a.q[v] = d->mq[d->mcur][v].as<double>(); a.din[v] = nullptr; a.w[v] = W.p(v); a.t[v] = T.p(v);
     }
     // (no epilogue arrays: t only)
     HIP_TRY(launch_rk_vjp(d->dev, a, d->stream));
-    HIP_TRY(download5(t, T, nb, d->stream));
+    HIP_TRY(download5(d, t, T));
     return NSEM_OK;
 }
 
@@ -826,7 +817,7 @@ int nsem_dg_residual_tlm(nsem_dg* d, const double* dq, double* L, double* dL) {
     std::vector<Field5> ws;
     HIP_TRY(workspace(d, 3, ws));
     const Field5 &TQ = ws[0], &Lout = ws[1], &TL = ws[2];
-    HIP_TRY(upload5(TQ, dq, nb, d->stream));
+    HIP_TRY(upload5(d, TQ, dq));
     RkArgs<double> a{};
     for (int v = 0; v < 5; v++) {
         a.q[v] = d->mq[d->mcur][v].as<double>();
@@ -837,12 +828,12 @@ int nsem_dg_residual_tlm(nsem_dg* d, const double* dq, double* L, double* dL) {
     a.b = 1.0;
     a.bdt = 1.0;   // out = L
     a.last = 0;
-    a.flag = d->flag.as<int>();
+    a.flag = d->flag();
     hipError_t e = launch_rk_stage<Dual<1>, double>(d->dev, a, d->stream);
     if (e == hipErrorInvalidValue) return nsem_fail(NSEM_EUNSUPPORTED, "element too large for the tangent-linear kernel");
     HIP_TRY(e);
-    HIP_TRY(download5(L, Lout, nb, d->stream));
-    HIP_TRY(download5(dL, TL, nb, d->stream));
+    HIP_TRY(download5(d, L, Lout));
+    HIP_TRY(download5(d, dL, TL));
     return NSEM_OK;
 }
 
@@ -854,7 +845,7 @@ int nsem_dg_rk3_tlm(nsem_dg* d, int32_t nsteps, double* dq) {
     std::vector<Field5> ws;
     HIP_TRY(workspace(d, 4, ws));
     const Field5 tq[2] = {ws[0], ws[1]}, td[2] = {ws[2], ws[3]};
-    HIP_TRY(upload5(tq[0], dq, nb, d->stream));
+    HIP_TRY(upload5(d, tq[0], dq));
     int tc = 0;
     for (int32_t s = 0; s < nsteps; s++) {
         DevBuf* qa = d->mq[d->mcur];
@@ -875,7 +866,7 @@ int nsem_dg_rk3_tlm(nsem_dg* d, int32_t nsteps, double* dq) {
             a.bdt = kB[stage] * d->dev.dt;
             a.last = stage == 2;
             a.check = stage == 2;
-            a.flag = d->flag.as<int>();
+            a.flag = d->flag();
             hipError_t e = launch_rk_stage<Dual<1>, double>(d->dev, a, d->stream);
             if (e == hipErrorInvalidValue)
                 return nsem_fail(NSEM_EUNSUPPORTED, "element too large for the tangent-linear kernel");
@@ -884,13 +875,14 @@ int nsem_dg_rk3_tlm(nsem_dg* d, int32_t nsteps, double* dq) {
         d->mcur = 1 - d->mcur;
         tc = 1 - tc;
     }
-    HIP_TRY(download5(dq, tq[tc], nb, d->stream));
+    bool finite = true;
+    HIP_TRY(download5(d, dq, tq[tc], &finite));
     if (nsteps > 0) {
         d->mol_valid = true;
         d->split_valid = false;
     }
     if (int rc0 = nsem_dg_take_flag(d, "non-finite state in the tangent-linear steps")) return rc0;
-    if (!all_finite(dq, 5 * nb)) return nsem_fail(NSEM_ENONFINITE, "non-finite tangent");
+    if (!finite) return nsem_fail(NSEM_ENONFINITE, "non-finite tangent");
     return NSEM_OK;
 }
 
@@ -898,8 +890,9 @@ int nsem_dg_rk3_tlm(nsem_dg* d, int32_t nsteps, double* dq) {
 
 // The adjoint sweep; with `seconds`, the device time from after the upload
 // of lam to before the download of the gradient (HIP events on the stream).
-static int rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, double* lam, double* seconds) {
-    if (!d || !lam || nsteps < 0 || checkpoint < 1) return nsem_fail(NSEM_EINVAL, "bad argument");
+static int rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, const double* lam, double* grad,
+                       double* seconds) {
+    if (!d || !lam || !grad || nsteps < 0 || checkpoint < 1) return nsem_fail(NSEM_EINVAL, "bad argument");
     int rc = check_adjoint_support(d);
     if (rc) return rc;
     if ((rc = nsem_dg_require_mol(d))) return rc;
@@ -915,7 +908,7 @@ static int rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, double* l
     const Field5* sd2 = sd1 + checkpoint;
     Field5 L = sd2[checkpoint];
     AdjointWork w{sd2[checkpoint + 1], sd2[checkpoint + 2]};
-    HIP_TRY(upload5(L, lam, nb, d->stream));
+    HIP_TRY(upload5(d, L, lam));
     if (seconds) HIP_TRY(hipEventRecord(d->ev0, d->stream));
     // one segment forward from its first state seg[0], recording each step's
     // state and stage increments; the state after the segment goes to `last`
@@ -984,21 +977,26 @@ static int rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, double* l
         HIP_TRY(hipEventElapsedTime(&ms, d->ev0, d->ev1));
         *seconds = ms * 1e-3;
     }
-    HIP_TRY(download5(lam, L, nb, d->stream));
+    bool finite = true;
+    HIP_TRY(download5(d, grad, L, &finite));
     if ((rc = nsem_dg_take_flag(d, "non-finite state in the adjoint's forward sweep"))) return rc;
-    if (!all_finite(lam, 5 * nb)) return nsem_fail(NSEM_ENONFINITE, "non-finite gradient");
+    if (!finite) return nsem_fail(NSEM_ENONFINITE, "non-finite gradient");
     return NSEM_OK;
 }
 
 extern "C" {
 
 int nsem_dg_rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, double* lam) {
-    return rk3_adjoint(d, nsteps, checkpoint, lam, nullptr);
+    return rk3_adjoint(d, nsteps, checkpoint, lam, lam, nullptr);
+}
+
+int nsem_dg_rk3_gradient(nsem_dg* d, int32_t nsteps, int32_t checkpoint, const double* lam, double* grad) {
+    return rk3_adjoint(d, nsteps, checkpoint, lam, grad, nullptr);
 }
 
 int nsem_dg_time_rk3_adjoint(nsem_dg* d, int32_t nsteps, int32_t checkpoint, double* lam, double* seconds) {
     if (!seconds) return nsem_fail(NSEM_EINVAL, "null argument");
-    return rk3_adjoint(d, nsteps, checkpoint, lam, seconds);
+    return rk3_adjoint(d, nsteps, checkpoint, lam, lam, seconds);
 }
 
 }  // extern "C"

@@ -64,6 +64,7 @@ int nsem_dg_create(const nsem_mesh* mesh, const nsem_euler_params* prm, const in
     HIP_TRY(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&d->ev0));
     HIP_TRY(hipEventCreate(&d->ev1));
+    HIP_TRY(d->pipe.init());
     hipStream_t s = d->stream;
 
     // boundary table: scalars must be zero-gradient on this path
@@ -416,8 +417,6 @@ int nsem_dg_create(const nsem_mesh* mesh, const nsem_euler_params* prm, const in
     if (prm->diffusion) HIP_TRY(d->grad.alloc(12 * nb * sizeof(double)));
     HIP_TRY(d->diag_slots.alloc(kDiagBlocks * 6 * sizeof(double)));
     HIP_TRY(d->diag_out.alloc(6 * sizeof(double)));
-    HIP_TRY(d->flag.alloc(sizeof(int)));
-    HIP_TRY(hipMemsetAsync(d->flag.p, 0, sizeof(int), s));
     HIP_TRY(d->gadj.alloc(ghost_rec.size() * 5 * npfm * sizeof(double)));
     HIP_TRY(hipStreamSynchronize(s));
     d->host_p_ref = pref;
@@ -463,7 +462,7 @@ int nsem_dg_create(const nsem_mesh* mesh, const nsem_euler_params* prm, const in
     dv.msurf_t = d->msurf_t.as<double>();
     dv.madj = d->madj.as<double>();
     dv.mgrad = d->mgrad.as<double>();
-    dv.flag = d->flag.as<int>();
+    dv.flag = d->flag();
     dv.nghost = (int)ghost_rec.size();
     dv.ghost_rec = d->ghost_rec.as<uint32_t>();
     dv.ghost_of = d->ghost_of.as<uint32_t>();
@@ -476,43 +475,31 @@ void nsem_dg_destroy(nsem_dg* d) { delete d; }
 
 int nsem_dg_set_state(nsem_dg* d, const double* rho, const double* U, const double* T, const double* p) {
     if (!d || !rho || !U || !T || !p) return nsem_fail(NSEM_EINVAL, "null argument");
-    const uint64_t nb = d->nb;
-    std::vector<double> ux(nb), uy(nb), uz(nb);
-    for (uint64_t n = 0; n < nb; n++) { ux[n] = U[3 * n]; uy[n] = U[3 * n + 1]; uz[n] = U[3 * n + 2]; }
-    const double* src[6] = {rho, ux.data(), uy.data(), uz.data(), T, p};
-    for (int v = 0; v < 6; v++)
-        HIP_TRY(hipMemcpyAsync(d->st[d->cur][v].p, src[v], nb * sizeof(double), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
+    DevBuf* A = d->st[d->cur];
+    PipeColumns c;
+    c.add(rho, A[0].as<double>());
+    c.add3(U, A[1].as<double>(), A[2].as<double>(), A[3].as<double>());
+    c.add(T, A[4].as<double>());
+    c.add(p, A[5].as<double>());
+    HIP_TRY(d->pipe.upload(c, d->nb, d->stream));
     // conserved perturbations for the method-of-lines path
-    const double T0 = d->prm.T0;
-    std::vector<double> q[5];
-    for (int v = 0; v < 5; v++) q[v].resize(nb);
-    for (uint64_t n = 0; n < nb; n++) {
-        const double rr = d->host_rho_ref[n];
-        q[0][n] = rho[n] - rr;
-        q[1][n] = rho[n] * ux[n];
-        q[2][n] = rho[n] * uy[n];
-        q[3][n] = rho[n] * uz[n];
-        q[4][n] = rho[n] * (T[n] + T0) - rr * T0;
-    }
-    for (int v = 0; v < 5; v++)
-        HIP_TRY(hipMemcpyAsync(d->mq[d->mcur][v].p, q[v].data(), nb * sizeof(double), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(hipMemsetAsync(d->flag.p, 0, sizeof(int), d->stream));
+    d->mol_valid = false;
+    if (int rc = nsem_dg_require_mol(d)) return rc;
     HIP_TRY(hipStreamSynchronize(d->stream));
-    d->split_valid = d->mol_valid = true;
+    *d->flag() = 0;
+    d->split_valid = true;
     return NSEM_OK;
 }
 
 int nsem_dg_set_conserved(nsem_dg* d, const double* rho_p, const double* m, const double* theta_p) {
     if (!d || !rho_p || !m || !theta_p) return nsem_fail(NSEM_EINVAL, "null argument");
-    const uint64_t nb = d->nb;
-    std::vector<double> mx(nb), my(nb), mz(nb);
-    for (uint64_t n = 0; n < nb; n++) { mx[n] = m[3 * n]; my[n] = m[3 * n + 1]; mz[n] = m[3 * n + 2]; }
-    const double* src[5] = {rho_p, mx.data(), my.data(), mz.data(), theta_p};
-    for (int v = 0; v < 5; v++)
-        HIP_TRY(hipMemcpyAsync(d->mq[d->mcur][v].p, src[v], nb * sizeof(double), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(hipMemsetAsync(d->flag.p, 0, sizeof(int), d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
+    DevBuf* q = d->mq[d->mcur];
+    PipeColumns c;
+    c.add(rho_p, q[0].as<double>());
+    c.add3(m, q[1].as<double>(), q[2].as<double>(), q[3].as<double>());
+    c.add(theta_p, q[4].as<double>());
+    HIP_TRY(d->pipe.upload(c, d->nb, d->stream));
+    *d->flag() = 0;
     d->mol_valid = true;
     d->split_valid = false;
     return NSEM_OK;
@@ -521,13 +508,12 @@ int nsem_dg_set_conserved(nsem_dg* d, const double* rho_p, const double* m, cons
 int nsem_dg_get_conserved(nsem_dg* d, double* rho_p, double* m, double* theta_p) {
     if (!d || !rho_p || !m || !theta_p) return nsem_fail(NSEM_EINVAL, "null argument");
     if (int rc = nsem_dg_require_mol(d)) return rc;
-    const uint64_t nb = d->nb;
-    std::vector<double> mx(nb), my(nb), mz(nb);
-    double* dst[5] = {rho_p, mx.data(), my.data(), mz.data(), theta_p};
-    for (int v = 0; v < 5; v++)
-        HIP_TRY(hipMemcpyAsync(dst[v], d->mq[d->mcur][v].p, nb * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
-    for (uint64_t n = 0; n < nb; n++) { m[3 * n] = mx[n]; m[3 * n + 1] = my[n]; m[3 * n + 2] = mz[n]; }
+    DevBuf* q = d->mq[d->mcur];
+    PipeColumns c;
+    c.add(rho_p, q[0].as<double>());
+    c.add3(m, q[1].as<double>(), q[2].as<double>(), q[3].as<double>());
+    c.add(theta_p, q[4].as<double>());
+    HIP_TRY(d->pipe.download(c, d->nb, d->stream));
     return NSEM_OK;
 }
 
@@ -539,21 +525,24 @@ int nsem_dg_get_state(nsem_dg* d, double* rho, double* U, double* T, double* p) 
         int rc = nsem_dg_get_conserved(d, rp.data(), m.data(), tp.data());
         if (rc) return rc;
         const double T0 = d->prm.T0, gam = d->prm.cp / d->prm.cv;
-        for (uint64_t n = 0; n < nb; n++) {
+        parallel_for(nb, [&](uint64_t nbeg, uint64_t nend) {
+        for (uint64_t n = nbeg; n < nend; n++) {
             const double rr = d->host_rho_ref[n];
             rho[n] = rr + rp[n];
             for (int c = 0; c < 3; c++) U[3 * n + c] = m[3 * n + c] / rho[n];
             T[n] = (tp[n] + rr * T0) / rho[n] - T0;
             p[n] = d->host_p_ref[n] * std::expm1(gam * std::log1p(tp[n] / (rr * T0)));
         }
+        });
         return NSEM_OK;
     }
-    std::vector<double> ux(nb), uy(nb), uz(nb);
-    double* dst[6] = {rho, ux.data(), uy.data(), uz.data(), T, p};
-    for (int v = 0; v < 6; v++)
-        HIP_TRY(hipMemcpyAsync(dst[v], d->st[d->cur][v].p, nb * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
-    for (uint64_t n = 0; n < nb; n++) { U[3 * n] = ux[n]; U[3 * n + 1] = uy[n]; U[3 * n + 2] = uz[n]; }
+    DevBuf* A = d->st[d->cur];
+    PipeColumns c;
+    c.add(rho, A[0].as<double>());
+    c.add3(U, A[1].as<double>(), A[2].as<double>(), A[3].as<double>());
+    c.add(T, A[4].as<double>());
+    c.add(p, A[5].as<double>());
+    HIP_TRY(d->pipe.download(c, nb, d->stream));
     return NSEM_OK;
 }
 
@@ -644,7 +633,7 @@ int rk3_steps_t(nsem_dg* d, int32_t nsteps, DevBuf (&dl)[2][5]) {
             a.bdt = kB[stage] * d->dev.dt;
             a.last = stage == 2;
             a.check = (stage == 2);
-            a.flag = d->flag.as<int>();
+            a.flag = d->flag();
             if (d->dev.diffusion) {
                 // the stage state's gradients for the viscous fluxes
                 R* grad = d->grad.as<R>();
@@ -692,12 +681,9 @@ int nsem_dg_require_split(nsem_dg* d) {
 }
 
 int nsem_dg_take_flag(nsem_dg* d, const char* what) {
-    int flag = 0;
-    HIP_TRY(hipMemcpyAsync(&flag, d->flag.p, sizeof(int), hipMemcpyDeviceToHost, d->stream));
     HIP_TRY(hipStreamSynchronize(d->stream));
-    if (!flag) return NSEM_OK;
-    HIP_TRY(hipMemsetAsync(d->flag.p, 0, sizeof(int), d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
+    if (!*d->flag()) return NSEM_OK;
+    *d->flag() = 0;
     return nsem_fail(NSEM_ENONFINITE, what);
 }
 

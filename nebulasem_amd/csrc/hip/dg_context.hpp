@@ -9,6 +9,7 @@
 #include "../status.hpp"
 #include "dg_common.hpp"
 #include "dg_kernels.hpp"
+#include "host_pipe.hpp"
 #include "nebulasem_amd.h"
 
 #define HIP_TRY(x)                                                                  \
@@ -51,7 +52,10 @@ struct nsem_dg {
     int cur = 0;
     // method-of-lines state: FP64 conserved perturbations (rho', m, Theta'),
     // double-buffered, and stage increments in FP64 and FP32
-    DevBuf mq[2][5], d64[2][5], d32[2][5], flag;
+    DevBuf mq[2][5], d64[2][5], d32[2][5];
+    // staging of the state transfers; its word is the non-finite flag, which
+    // the kernels write over the link (only when it is raised)
+    nsem::HostPipe pipe;
     // diagnostics: g.x per node, block partials, result
     DevBuf gh, diag_slots, diag_out;
     // strong gradients of U and theta of the viscous split step [12][nb]
@@ -69,6 +73,7 @@ struct nsem_dg {
     double prof_ms[4] = {0, 0, 0, 0};
     uint64_t prof_n[4] = {0, 0, 0, 0};
     std::vector<double> host_p_ref, host_rho_ref;
+    int* flag() const { return pipe.word(); }
     ~nsem_dg() {
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);

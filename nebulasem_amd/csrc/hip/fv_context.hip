@@ -18,6 +18,7 @@
 #include "../mesh_access.hpp"
 #include "../status.hpp"
 #include "fv_kernels.hpp"
+#include "host_pipe.hpp"
 #include "nebulasem_amd.h"
 
 using namespace nsem;
@@ -71,12 +72,25 @@ struct nsem_fv {
     Buf x, r, z, p, Ap, x32, r32, z32, p32, Ap32, e32, b32, y64, slots, sc, tmp, posts, faces;
     FvBoxes boxes64, boxes32;            // the on-chip conjugate gradient's work-groups
     std::vector<int32_t> patch_kind;
+    HostPipe pipe;   // staging of the cell arrays
     ~nsem_fv() {
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
+
+// One array of n doubles between the caller and the device; both wait.
+static hipError_t put_cells(nsem_fv* d, void* dev, const double* host, uint64_t n) {
+    PipeColumns c;
+    c.add(host, (double*)dev);
+    return d->pipe.upload(c, n, d->stream);
+}
+static hipError_t get_cells(nsem_fv* d, double* host, void* dev, uint64_t n) {
+    PipeColumns c;
+    c.add(host, (double*)dev);
+    return d->pipe.download(c, n, d->stream);
+}
 
 static int fv_build(nsem_fv& d, const Geometry& g, size_t npatch, const std::vector<double>& ap,
                     const std::vector<double>& ano, const std::vector<double>& ann, const std::vector<double>& subc,
@@ -104,6 +118,7 @@ int nsem_fv_create(const nsem_mesh* mesh, const double* mu, const int32_t* bc_ki
     HIP_TRY(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&d->ev0));
     HIP_TRY(hipEventCreate(&d->ev1));
+    HIP_TRY(d->pipe.init());
     hipStream_t s = d->stream;
 
     // couplings ano = ann = fD * cds(mu)
@@ -360,6 +375,7 @@ int nsem_fv_create_coeffs(const nsem_mesh* mesh, const double* ap, const double*
     HIP_TRY(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&d->ev0));
     HIP_TRY(hipEventCreate(&d->ev1));
+    HIP_TRY(d->pipe.init());
     d->nghost = nc - n;
     std::vector<double> vap(ap, ap + nc), vano(ano, ano + nf), vann(ann, ann + nf), subc(n, 0.0);
     // couplings to ghost cells: the caller has folded the boundary
@@ -388,7 +404,7 @@ int nsem_fv_set_rhs_divergence(nsem_fv* d, const double* U, const int32_t* bc_ki
                                int32_t nboundaries) {
     if (!d || !U || !bc_kind || !bc_value || nboundaries < 0) return nsem_fail(NSEM_EINVAL, "bad argument");
     hipStream_t s = d->stream;
-    HIP_TRY(hipMemcpyAsync(d->U.p, U, 3 * d->n * sizeof(double), hipMemcpyHostToDevice, s));
+    HIP_TRY(put_cells(d, d->U.p, U, 3 * d->n));
     if (nboundaries) {
         HIP_TRY(hipMemcpyAsync(d->ubc_kind.p, bc_kind, nboundaries * sizeof(int32_t), hipMemcpyHostToDevice, s));
         HIP_TRY(hipMemcpyAsync(d->ubc_value.p, bc_value, 3 * nboundaries * sizeof(double), hipMemcpyHostToDevice, s));
@@ -400,37 +416,37 @@ int nsem_fv_set_rhs_divergence(nsem_fv* d, const double* U, const int32_t* bc_ki
 
 int nsem_fv_set_rhs(nsem_fv* d, const double* su) {
     if (!d || !su) return nsem_fail(NSEM_EINVAL, "null argument");
-    HIP_TRY(hipMemcpyAsync(d->su.p, su, d->n * sizeof(double), hipMemcpyHostToDevice, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
+    HIP_TRY(put_cells(d, d->su.p, su, d->n));
     return NSEM_OK;
 }
 
 int nsem_fv_get_rhs(nsem_fv* d, double* su) {
     if (!d || !su) return nsem_fail(NSEM_EINVAL, "null argument");
-    HIP_TRY(hipMemcpyAsync(su, d->su.p, d->n * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    HIP_TRY(hipStreamSynchronize(d->stream));
+    HIP_TRY(get_cells(d, su, d->su.p, d->n));
+    return NSEM_OK;
+}
+
+int nsem_fv_corrected_velocity(nsem_fv* d, const double* p, const double* U, double* out) {
+    if (!d || !p || !U || !out) return nsem_fail(NSEM_EINVAL, "null argument");
+    hipStream_t s = d->stream;
+    HIP_TRY(put_cells(d, d->y64.p, p, d->n));
+    HIP_TRY(put_cells(d, d->U.p, U, 3 * d->n));
+    HIP_TRY(fv_gradcorr(d->div, d->y64.as<double>(), d->pg_kind.as<int32_t>(), d->pg_off.as<double>(),
+                        d->cV.as<double>(), d->nghost, d->U.as<double>(), s));
+    HIP_TRY(get_cells(d, out, d->U.p, 3 * d->n));
     return NSEM_OK;
 }
 
 int nsem_fv_correct_velocity(nsem_fv* d, const double* p, double* U) {
-    if (!d || !p || !U) return nsem_fail(NSEM_EINVAL, "null argument");
-    hipStream_t s = d->stream;
-    HIP_TRY(hipMemcpyAsync(d->y64.p, p, d->n * sizeof(double), hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(d->U.p, U, 3 * d->n * sizeof(double), hipMemcpyHostToDevice, s));
-    HIP_TRY(fv_gradcorr(d->div, d->y64.as<double>(), d->pg_kind.as<int32_t>(), d->pg_off.as<double>(),
-                        d->cV.as<double>(), d->nghost, d->U.as<double>(), s));
-    HIP_TRY(hipMemcpyAsync(U, d->U.p, 3 * d->n * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return NSEM_OK;
+    return nsem_fv_corrected_velocity(d, p, U, U);
 }
 
 int nsem_fv_apply(nsem_fv* d, const double* x, double* y) {
     if (!d || !x || !y) return nsem_fail(NSEM_EINVAL, "null argument");
     hipStream_t s = d->stream;
-    HIP_TRY(hipMemcpyAsync(d->x.p, x, d->n * sizeof(double), hipMemcpyHostToDevice, s));
+    HIP_TRY(put_cells(d, d->x.p, x, d->n));
     HIP_TRY(fv_apply(d->A64, d->x.as<double>(), d->y64.as<double>(), s));
-    HIP_TRY(hipMemcpyAsync(y, d->y64.p, d->n * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(get_cells(d, y, d->y64.p, d->n));
     return NSEM_OK;
 }
 
@@ -486,7 +502,7 @@ extern "C" int nsem_fv_solve(nsem_fv* d, double* x_io, int32_t mode, double tol,
     std::memset(res, 0, sizeof(*res));
     hipStream_t s = d->stream;
     const uint64_t n = d->n;
-    HIP_TRY(hipMemcpyAsync(d->x.p, x_io, n * sizeof(double), hipMemcpyHostToDevice, s));
+    HIP_TRY(put_cells(d, d->x.p, x_io, n));
     HIP_TRY(hipEventRecord(d->ev0, s));
     CgScalars hs{};
     int rc = NSEM_OK;
@@ -545,8 +561,7 @@ extern "C" int nsem_fv_solve(nsem_fv* d, double* x_io, int32_t mode, double tol,
     HIP_TRY(fv_norm2<double>(n, d->su.as<double>(), tmp2 + 1, d->slots.as<double>(), s));
     HIP_TRY(hipMemcpyAsync(&rr, tmp2, sizeof(double), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipMemcpyAsync(&bb, tmp2 + 1, sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(x_io, d->x.p, n * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(get_cells(d, x_io, d->x.p, n));
     res->res_true = bb > 0 ? std::sqrt(rr / bb) : 0;
     res->breakdown = hs.breakdown;
     (void)0;

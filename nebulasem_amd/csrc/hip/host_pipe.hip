@@ -1,0 +1,198 @@
+// Host <-> device copies of node arrays, as the C-ABI's state calls need
+// them: the caller's pageable memory, vectors interleaved there and split by
+// component on the device.
+//
+// What bounds it is the host side: the first write to each page of the
+// caller's memory and one core's copy rate, far below the link.  So the rows
+// go in chunks through pinned staging memory: a kernel reads or writes the
+// staging memory over the link (interleaving on the way) while up to eight
+// threads copy the chunk before between it and the caller's memory.
+#include "host_pipe.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <thread>
+#include <vector>
+
+#include "../host/parallel.hpp"
+
+namespace nsem {
+
+namespace {
+
+struct KernelColumns {
+    int comps[PipeColumns::kMax];
+    double* dev[PipeColumns::kMax][3];
+};
+
+// blockIdx.y: column.  Consecutive threads take consecutive staged words, so
+// the accesses over the link are whole lines.
+template <bool UP>
+__global__ void __launch_bounds__(256) stage_kernel(KernelColumns c, uint64_t first, uint32_t rows, double* stage,
+                                                    int* bad) {
+    const int g = blockIdx.y;
+    size_t off = 0;
+    for (int k = 0; k < g; k++) off += (size_t)c.comps[k] * rows;
+    const uint32_t words = rows * (uint32_t)c.comps[g];
+    double* st = stage + off;
+    bool wrong = false;
+    for (uint32_t w = blockIdx.x * 256 + threadIdx.x; w < words; w += gridDim.x * 256) {
+        double* d;
+        if (c.comps[g] == 1) {
+            d = c.dev[g][0] + first + w;
+        } else {
+            const uint32_t row = w / 3, k = w - 3 * row;
+            d = (k == 0 ? c.dev[g][0] : k == 1 ? c.dev[g][1] : c.dev[g][2]) + first + row;
+        }
+        if constexpr (UP) {
+            *d = st[w];
+        } else {
+            const double v = *d;
+            st[w] = v;
+            wrong = wrong || !isfinite(v);
+        }
+    }
+    if (!UP && bad && wrong) *bad = 1;
+}
+
+// Below kThreaded bytes the calling thread copies alone: a new thread can wait
+// milliseconds for a core that another pool's threads spin on.  Below kOne a
+// copy is one chunk, else chunks of a twelfth, three of them in flight.
+constexpr size_t kThreaded = 8u << 20, kOne = 512u << 10;
+
+}  // namespace
+
+HostPipe::~HostPipe() {
+    for (hipEvent_t e : ev_)
+        if (e) (void)hipEventDestroy(e);
+    if (stage_) (void)hipHostFree(stage_);
+    if (word_) (void)hipHostFree(word_);
+}
+
+hipError_t HostPipe::init() {
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&word_), 2 * sizeof(int), hipHostMallocDefault);
+    if (e != hipSuccess) return e;
+    word_[0] = word_[1] = 0;
+    for (hipEvent_t& v : ev_)
+        if ((e = hipEventCreateWithFlags(&v, hipEventDisableTiming)) != hipSuccess) return e;
+    return hipSuccess;
+}
+
+hipError_t HostPipe::upload(const PipeColumns& c, uint64_t count, hipStream_t s) {
+    return run(c, count, s, true, nullptr);
+}
+
+hipError_t HostPipe::download(const PipeColumns& c, uint64_t count, hipStream_t s, bool* finite) {
+    if (!finite) return run(c, count, s, false, nullptr);
+    word_[1] = 0;
+    const hipError_t e = run(c, count, s, false, word_ + 1);
+    *finite = word_[1] == 0;
+    return e;
+}
+
+hipError_t HostPipe::run(const PipeColumns& c, uint64_t count, hipStream_t s, bool up, int* bad) {
+    if (count == 0 || c.n == 0) return hipStreamSynchronize(s);
+    size_t row = 0;
+    KernelColumns kc{};
+    for (int g = 0; g < c.n; g++) {
+        kc.comps[g] = c.comps[g];
+        row += c.comps[g] * sizeof(double);
+        for (int k = 0; k < 3; k++) kc.dev[g][k] = c.dev[g][k];
+    }
+    const size_t total = row * count;
+    const unsigned threads =
+        total < kThreaded ? 1 : (unsigned)std::min<size_t>({8, host_threads(), total >> 20});
+    const size_t bytes = std::min(kChunk, std::max<size_t>(256u << 10, total / 12));
+    const uint64_t chunk = total < kOne ? count : std::min<uint64_t>(count, std::max<uint64_t>(1, bytes / row));
+    const uint64_t chunks = (count + chunk - 1) / chunk;
+    const int slots = (int)std::min<uint64_t>(kSlots, chunks);
+    const size_t need = row * chunk * slots;
+    hipError_t e;
+    if (bytes_ < need) {
+        if (stage_) {
+            // (a copy has always been waited for when run() returns)
+            (void)hipHostFree(stage_);
+            stage_ = nullptr;
+            bytes_ = 0;
+        }
+        if ((e = hipHostMalloc(reinterpret_cast<void**>(&stage_), need, hipHostMallocDefault)) != hipSuccess) {
+            stage_ = nullptr;
+            return e;
+        }
+        bytes_ = need;
+    }
+    auto rows_of = [&](uint64_t k) { return (uint32_t)std::min<uint64_t>(chunk, count - k * chunk); };
+    auto slot_of = [&](uint64_t k) { return stage_ + (size_t)(k % slots) * (row / sizeof(double)) * chunk; };
+    auto launch = [&](uint64_t k) -> hipError_t {
+        const uint32_t rows = rows_of(k);
+        const dim3 grid((unsigned)std::min<uint64_t>(512, (3ull * rows + 255) / 256), (unsigned)c.n);
+        if (up) hipLaunchKernelGGL(stage_kernel<true>, grid, dim3(256), 0, s, kc, k * chunk, rows, slot_of(k), bad);
+        else hipLaunchKernelGGL(stage_kernel<false>, grid, dim3(256), 0, s, kc, k * chunk, rows, slot_of(k), bad);
+        const hipError_t err = hipGetLastError();
+        return err != hipSuccess ? err : hipEventRecord(ev_[k % slots], s);
+    };
+    // thread t's share of chunk k, column by column
+    auto copy = [&](uint64_t k, unsigned t, unsigned of) {
+        const size_t rows = rows_of(k);
+        double* st = slot_of(k);
+        for (int g = 0; g < c.n; g++) {
+            const size_t words = rows * c.comps[g], a = words * t / of, b = words * (t + 1) / of;
+            double* h = c.host[g] + (size_t)k * chunk * c.comps[g] + a;
+            if (up) std::memcpy(st + a, h, (b - a) * sizeof(double));
+            else std::memcpy(h, st + a, (b - a) * sizeof(double));
+            st += words;
+        }
+    };
+    if (threads == 1 && chunks == 1) {
+        if (up) copy(0, 0, 1);
+        if ((e = launch(0)) != hipSuccess) return e;
+        if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+        if (!up) copy(0, 0, 1);
+        return hipSuccess;
+    }
+    // Each chunk is copied in 2 * threads pieces, claimed in order; `open` is
+    // the number of pieces that may be claimed, `done` of those finished.  A
+    // thread that is late finds its work done: it is not waited for.
+    const unsigned per = threads > 1 ? 2 * threads : 1;
+    std::atomic<uint64_t> open{0}, next{0}, done{0};
+    std::atomic<bool> stop{false};
+    auto claim = [&]() -> bool {
+        uint64_t i = next.load(std::memory_order_relaxed);
+        do {
+            if (i >= open.load(std::memory_order_acquire)) return false;
+        } while (!next.compare_exchange_weak(i, i + 1, std::memory_order_acq_rel));
+        copy(i / per, (unsigned)(i % per), per);
+        done.fetch_add(1, std::memory_order_acq_rel);
+        return true;
+    };
+    std::vector<std::thread> team;
+    try {
+        if (threads > 1) team.reserve(threads);
+        for (unsigned t = 1; t < threads; t++)
+            team.emplace_back([&] {
+                while (!stop.load(std::memory_order_relaxed))
+                    if (!claim()) std::this_thread::yield();
+            });
+    } catch (...) {
+        // no further thread to be had: those there are will do
+    }
+    e = hipSuccess;
+    if (!up)
+        for (int k = 0; k < slots && e == hipSuccess; k++) e = launch(k);
+    for (uint64_t k = 0; k < chunks && e == hipSuccess; k++) {
+        if (!up || k >= (uint64_t)slots) e = hipEventSynchronize(ev_[k % slots]);
+        if (e != hipSuccess) break;
+        open.store((k + 1) * per, std::memory_order_release);
+        while (claim()) {}
+        while (done.load(std::memory_order_acquire) < (k + 1) * per) std::this_thread::yield();
+        if (up) e = launch(k);
+        else if (k + slots < chunks) e = launch(k + slots);
+    }
+    stop = true;
+    for (auto& x : team) x.join();
+    const hipError_t es = hipStreamSynchronize(s);
+    return e != hipSuccess ? e : es;
+}
+
+}  // namespace nsem

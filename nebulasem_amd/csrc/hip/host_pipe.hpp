@@ -1,0 +1,53 @@
+// Node arrays between the caller's memory and the device.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+
+namespace nsem {
+
+// Columns of one transfer: `count` rows each, column g of comps[g] (1 or 3)
+// values a row, interleaved in host[g], one device array per component.
+struct PipeColumns {
+    static constexpr int kMax = 6;
+    int n = 0;
+    int comps[kMax] = {};
+    double* host[kMax] = {};
+    double* dev[kMax][3] = {};
+    void add(const double* h, double* d) {
+        host[n] = const_cast<double*>(h); comps[n] = 1; dev[n][0] = d; n++;
+    }
+    void add3(const double* h, double* x, double* y, double* z) {
+        host[n] = const_cast<double*>(h); comps[n] = 3;
+        dev[n][0] = x; dev[n][1] = y; dev[n][2] = z; n++;
+    }
+};
+
+// A handle's pinned staging memory (at most kSlots chunks) and a word of
+// pinned memory that kernels may write.  Not shared between handles; freed
+// with its handle.
+class HostPipe {
+public:
+    static constexpr int kSlots = 3;
+    static constexpr size_t kChunk = 4u << 20;
+    HostPipe() = default;
+    HostPipe(const HostPipe&) = delete;
+    HostPipe& operator=(const HostPipe&) = delete;
+    ~HostPipe();
+    hipError_t init();
+    int* word() const { return word_; }
+    // Both wait for the copy.  `finite` (download): set to false when a
+    // value is NaN or infinite.
+    hipError_t upload(const PipeColumns& c, uint64_t count, hipStream_t s);
+    hipError_t download(const PipeColumns& c, uint64_t count, hipStream_t s, bool* finite = nullptr);
+
+private:
+    hipError_t run(const PipeColumns& c, uint64_t count, hipStream_t s, bool up, int* bad);
+    double* stage_ = nullptr;
+    size_t bytes_ = 0;
+    int* word_ = nullptr;      // [0] the caller's, [1] download's
+    hipEvent_t ev_[kSlots] = {};
+};
+
+}  // namespace nsem
