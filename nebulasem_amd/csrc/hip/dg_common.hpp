@@ -60,6 +60,7 @@ struct DgDev {
     // binomial(gamma, k), k = 1..8: the FP64 series of (1 + x)^gamma - 1
     // (kernel arguments, so the kernels read them from scalar registers)
     double ppc[8];
+    float ppc32[6];                   // k = 1..6 for the FP32 series
     double g[3];
     int buoyancy;
     const double* JcV;                // [9][nb]
@@ -68,9 +69,22 @@ struct DgDev {
     const float* cV32;                // [nb]
     const double* p_ref;              // [nb]
     const double* rho_ref;            // [nb]
+    const float* p_ref32;             // FP32 copies
+    const float* rho_ref32;
     const EFace* eface;               // [nelem*6]
+    // [nelem*6][4]: outward unit normal of the element's face and its scale:
+    // the facet's area, in FP64 on affine elements times 2 / cell volume (|Jinv| of the
+    // face's direction), so that a flux per unit area is scaled to its share
+    // of L(q) times w_end
+    const double* fnorm;
+    const float* fnorm32;
+    int yfaces;                       // 0: no face of groups 2 and 3 is present
     const double* gFN;                // [nfacets*3]
     const double* D[3];               // [n*n] per direction
+    // the three directions' D one after the other (Dm), and D[t*n+i] w_t / w_i
+    // (DWm); FP32 copy of the first
+    const double *Dm, *DWm;
+    const float* Dm32;
     const double* w[3];               // [n] per direction
     const BcTable* bc;
     // artificial viscosity of the split step (euler.cpp:188-190): mu =

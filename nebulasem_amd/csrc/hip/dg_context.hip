@@ -361,7 +361,45 @@ int nsem_dg_create(const nsem_mesh* mesh, const nsem_euler_params* prm, const in
     std::vector<double> gfn(3 * (size_t)g.nfacets);
     for (Int f = 0; f < g.nfacets; f++)
         for (int c = 0; c < 3; c++) gfn[3 * (size_t)f + c] = lm.fn[f][c];
+    // outward unit normals and scales of the elements' faces
+    std::vector<double> fnorm((size_t)g.nbcs * 24, 0.0);
+    int yfaces = 0;
+    for (size_t r = 0; r < ef.size(); r++) {
+        const uint32_t m = ef[r].meta;
+        if (!((m >> 4) & 1)) continue;
+        const int grp = (int)(r % 6), dir = grp < 2 ? 2 : grp < 4 ? 1 : 0;
+        if (dir == 1) yfaces = 1;
+        const double* nv = &gfn[3 * (size_t)ef[r].facet];
+        const double len = std::sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]);
+        const double sg = (m >> 3) & 1 ? 1.0 : -1.0;
+        for (int c = 0; c < 3; c++) fnorm[4 * r + c] = sg * nv[c] / len;
+        fnorm[4 * r + 3] = all_affine ? len * 2 / lm.cv[r / 6] : len;
+    }
+    std::vector<float> fnorm32(fnorm.begin(), fnorm.end());
+    // (the FP32 form takes the per-node metric: the facet's area)
+    for (size_t r = 0; r < ef.size(); r++) {
+        const double* nv = &gfn[3 * (size_t)ef[r].facet];
+        if ((ef[r].meta >> 4) & 1) fnorm32[4 * r + 3] = (float)std::sqrt(nv[0] * nv[0] + nv[1] * nv[1] + nv[2] * nv[2]);
+    }
+    std::vector<float> pref32(pref.begin(), pref.end()), rref32(rref.begin(), rref.end());
     hipError_t e;
+    if ((e = upload(d->fnorm, fnorm, s)) != hipSuccess || (e = upload(d->fnorm32, fnorm32, s)) != hipSuccess ||
+        (e = upload(d->p_ref32, pref32, s)) != hipSuccess || (e = upload(d->rho_ref32, rref32, s)) != hipSuccess)
+        return nsem_fail(NSEM_EDEVICE, std::string("upload: ") + hipGetErrorString(e));
+    std::vector<double> Dm, DWm;
+    for (int dir = 0; dir < 3; dir++) {
+        const std::vector<double>&D = g.basis[dir].dpsi, &w = g.basis[dir].w;
+        const size_t n1 = w.size();
+        for (size_t t = 0; t < n1; t++)
+            for (size_t i = 0; i < n1; i++) {
+                Dm.push_back(D[t * n1 + i]);
+                DWm.push_back(D[t * n1 + i] * w[t] / w[i]);
+            }
+    }
+    const std::vector<float> Dm32(Dm.begin(), Dm.end());
+    if ((e = upload(d->Dm, Dm, s)) != hipSuccess || (e = upload(d->DWm, DWm, s)) != hipSuccess ||
+        (e = upload(d->Dm32, Dm32, s)) != hipSuccess)
+        return nsem_fail(NSEM_EDEVICE, std::string("upload: ") + hipGetErrorString(e));
     if ((e = upload(d->JcV, JcV, s)) != hipSuccess || (e = upload(d->cV, cV, s)) != hipSuccess ||
         (e = upload(d->JcV32, JcV32, s)) != hipSuccess || (e = upload(d->cV32, cV32, s)) != hipSuccess ||
         (e = upload(d->p_ref, pref, s)) != hipSuccess || (e = upload(d->rho_ref, rref, s)) != hipSuccess ||
@@ -428,11 +466,17 @@ int nsem_dg_create(const nsem_mesh* mesh, const nsem_euler_params* prm, const in
     dv.dt = prm->dt; dv.P0 = prm->P0; dv.T0 = prm->T0; dv.R = R; dv.gamma = gam; dv.cp = prm->cp;
     dv.ppc[0] = gam;
     for (int k = 1; k < 8; k++) dv.ppc[k] = dv.ppc[k - 1] * (gam - k) / (k + 1);
+    for (int k = 0; k < 6; k++) dv.ppc32[k] = (float)dv.ppc[k];
     for (int c = 0; c < 3; c++) dv.g[c] = prm->gravity[c];
     dv.buoyancy = prm->buoyancy;
     dv.JcV = d->JcV.as<double>(); dv.cV = d->cV.as<double>();
     dv.JcV32 = d->JcV32.as<float>(); dv.cV32 = d->cV32.as<float>();
     dv.p_ref = d->p_ref.as<double>(); dv.rho_ref = d->rho_ref.as<double>();
+    dv.p_ref32 = d->p_ref32.as<float>(); dv.rho_ref32 = d->rho_ref32.as<float>();
+    dv.fnorm = d->fnorm.as<double>(); dv.fnorm32 = d->fnorm32.as<float>();
+    dv.yfaces = yfaces;
+    dv.Dm = d->Dm.as<double>(); dv.DWm = d->DWm.as<double>();
+    dv.Dm32 = d->Dm32.as<float>();
     dv.eface = d->eface.as<EFace>(); dv.gFN = d->gFN.as<double>();
     for (int dir = 0; dir < 3; dir++) { dv.D[dir] = d->D[dir].as<double>(); dv.w[dir] = d->w[dir].as<double>(); }
     dv.bc = d->bc.as<BcTable>();

@@ -41,7 +41,9 @@ struct nsem_dg {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     uint64_t nb = 0;
     // geometry
-    DevBuf JcV, cV, JcV32, cV32, p_ref, rho_ref, eface, gFN, D[3], w[3], bc, emet, wnode;
+    DevBuf JcV, cV, JcV32, cV32, p_ref, rho_ref, p_ref32, rho_ref32, eface, fnorm, fnorm32, gFN, D[3], Dm, DWm, Dm32,
+        w[3], bc,
+        emet, wnode;
     // 2:1 non-conforming faces (empty on conforming meshes)
     DevBuf mort, mort_fine, mort_fms, mort_w, mort_bg, psiRef[3], psiCor[3], cslot, mphi, msurf, mphi_t, msurf_t,
         madj, mgrad;

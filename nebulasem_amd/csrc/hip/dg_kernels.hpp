@@ -79,7 +79,7 @@ size_t rk_vjp_lds_bytes(int nx, int ny, int nz, int epb, bool prims_in_lds);
 
 
 // LDS of the RK stage kernel, in values of the residual type: per element
-// max(15 flux rows x NP, 10 padded primitive rows + 5 face-flux rows x NFN),
+// max(15 flux rows x NP, 10 padded trace rows + 5 face-flux rows x NFN),
 // plus the three derivative matrices once per work-group.
 __host__ __device__ inline int rk_prim_stride(int np) { return np + (np + 7) / 8; }
 __host__ __device__ inline int rk_prim_slot(int node) { return node + (node >> 3); }

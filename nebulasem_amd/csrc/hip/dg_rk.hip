@@ -1,440 +1,18 @@
-// Method-of-lines dGSEM Euler residual fused with an SSP-RK3 stage
-// (Shu-Osher form, written as increments over the step's base state):
-//
-//   d1 = dt L(q)            d2 = (d1 + dt L(q + d1)) / 4
-//   d3 = 2 (d2 + dt L(q + d2)) / 3                  q^{n+1} = q + d3
-//
-// State: conserved perturbations over the FP64 hydrostatic background,
-//   rho' = rho - rho_ref,  m = rho U,  Theta' = rho theta - rho_ref T0.
-// Spatial operator: the reference's (divf + rusanov + div_flux + src,
-// field.h:2927-2943, 3085-3117, 3416-3478, 3711-3723) with all fluxes
-// evaluated at one state: F_rho = m, F_m = m (x) U + p' I, F_Theta = m theta,
-// lambda = (avg|U| + avg sqrt(gamma R theta)) / 2, normal-only momentum
-// dissipation, buoyancy (rho - rho_ref) g.  p' = p_ref expm1(gamma
-// log1p(Theta'/(rho_ref T0))) is the exact p(rho theta) - p_ref without the
-// cancellation, so the flux never touches the background's hydrostatic
-// balance.
-//
-// Template parameters: R the arithmetic type of the residual (double, or
-// float for the FP32-perturbation form), S the storage type of the stage
-// increments.  The base state and the final accumulation q + d3 are FP64 in
-// both forms; the background is FP64 and converted once per node.
-//
-// One work-group per element (NP threads, NP = 512 at N = 7): contravariant
-// fluxes of the 5 equations staged in LDS (15 x NP values), transposed 1-D
-// derivative along the three GLL lines, Rusanov surface terms from the
-// neighbour traces (global, L2/MALL resident), update fused.  Work-groups are
-// mapped to elements XCD-contiguously so face neighbours share an L2.
-// The method-of-lines path has no bit-level counterpart in the reference, so
-// products and sums are fused into FMAs here, in the headers' inline physics
-// too (the split reference-order kernels keep the build-wide
-// -ffp-contract=off).
-#pragma clang fp contract(fast)
+// Method-of-lines dGSEM Euler: the gradient and 2:1 mortar passes of a stage,
+// and the dispatch of the stage kernel (dg_rk_stage.hpp) by element shape.
+#include "dg_rk_stage.hpp"
 
-#include "dg_kernels.hpp"
-#include "dg_physics.hpp"
+NSEM_RK_SHAPE_(extern, 8, 8, 8)
+NSEM_RK_SHAPE_(extern, 7, 7, 7)
+NSEM_RK_SHAPE_(extern, 6, 6, 6)
+NSEM_RK_SHAPE_(extern, 5, 5, 5)
+NSEM_RK_SHAPE_(extern, 4, 4, 4)
+NSEM_RK_SHAPE_(extern, 5, 1, 5)
+NSEM_RK_SHAPE_(extern, 6, 1, 6)
+NSEM_RK_SHAPE_(extern, 7, 1, 7)
+NSEM_RK_SHAPE_(extern, 0, 0, 0)
 
 namespace nsem {
-
-namespace {
-
-// Stores of the stage output bypass the caches' retention (non-temporal):
-// they are not read again in this launch, and the L2 keeps the neighbour
-// traces instead.
-template <bool O32, typename T>
-__device__ __forceinline__ void stn(T* base, uint64_t i, T v) {
-    if constexpr (O32)
-        __builtin_nontemporal_store(v, reinterpret_cast<T*>(reinterpret_cast<char*>(base) + byte_off(i, sizeof(T))));
-    else
-        __builtin_nontemporal_store(v, base + i);
-}
-
-// Increment of variable v at node n (DIN: the stage has one; a compile-time
-// choice, so the loads carry no null-pointer branches between them).
-template <bool O32, bool DIN, typename S>
-__device__ __forceinline__ double ld_delta(const S* d, uint64_t i) {
-    if constexpr (DIN) return (double)ldn<O32>(d, i);
-    else return 0.0;
-}
-
-// State q + d_in of variable v at node n in the residual type (with its
-// tangent for the tangent-linear instantiation).
-template <typename R, typename S, bool O32, bool DIN>
-__device__ __forceinline__ R load_state(const RkArgs<S>& a, int v, uint64_t n) {
-    const double x = ldn<O32>(a.q[v], n) + ld_delta<O32, DIN>(a.din[v], n);
-    if constexpr (is_dual<R>::value) {
-        R r(x);
-        r.d[0] = ldn<O32>(a.tq[v], n) + ld_delta<O32, DIN>(a.tdin[v], n);
-        return r;
-    } else {
-        return (R)x;
-    }
-}
-
-}  // namespace
-
-// Everything one face-node task reads from global memory, gathered before
-// the volume term so that its latency overlaps the element's own loads:
-// the face entry, the weighted facet normal and the neighbour's state (on a
-// boundary or absent face the owner's own face node is read instead, so the
-// loads need no branch; only its background density is used there).
-template <typename R>
-struct FaceTask {
-    uint32_t meta;
-    int g, fa, fb, fnode;
-    uint64_t node;    // the node the state was read from (neighbour, or own on a boundary)
-    R nv[3];
-    R rp, m[3], tp, rref, pref;
-};
-
-template <typename R, typename S, bool O32, bool DIN>
-__device__ __forceinline__ void prepare_face_task(const DgDev& d, const RkArgs<S>& a, uint32_t e, int t,
-                                                  int NX, int NY, int NZ, FaceTask<R>& F) {
-    face_task(t, NX, NY, NZ, F.g, F.fa, F.fb, F.fnode);
-    // one 12-byte load of the face entry (facet, other, meta)
-    const uint3 efv = *reinterpret_cast<const uint3*>(d.eface + (size_t)e * 6 + F.g);
-    const EFace ef{efv.x, efv.y, efv.z};
-    F.meta = ef.meta;
-    const bool present = (ef.meta >> 4) & 1;
-    const bool interior = present && !((ef.meta >> 5) & 1);
-    const bool own = (ef.meta >> 3) & 1;
-    const int og = ef.meta & 7;
-    // facet-node weight w_a w_b / 4 in the owner's face layout (face_weight)
-    const int wg = own ? F.g : og;
-    const double* wa = wg < 4 ? d.w[0] : d.w[1];
-    const double* wb = wg < 2 ? d.w[1] : d.w[2];
-    const double wgt = wa[F.fa] * wb[F.fb] / 4;
-    const size_t f3 = 3 * (size_t)(present ? ef.facet : 0);
-    F.nv[0] = (R)(d.gFN[f3] * wgt);
-    F.nv[1] = (R)(d.gFN[f3 + 1] * wgt);
-    F.nv[2] = (R)(d.gFN[f3 + 2] * wgt);
-    const uint64_t m = interior ? face_node(ef.other, og, F.fa, F.fb, NX, NY, NZ)
-                                : (uint64_t)e * (NX * NY * NZ) + F.fnode;
-    F.node = m;
-    F.rp = load_state<R, S, O32, DIN>(a, 0, m);
-    F.m[0] = load_state<R, S, O32, DIN>(a, 1, m);
-    F.m[1] = load_state<R, S, O32, DIN>(a, 2, m);
-    F.m[2] = load_state<R, S, O32, DIN>(a, 3, m);
-    F.tp = load_state<R, S, O32, DIN>(a, 4, m);
-    F.rref = (R)ldn<O32>(d.rho_ref, m);
-    F.pref = (R)ldn<O32>(d.p_ref, m);
-}
-
-// Ghost-node gradients of the viscous terms, as the split step forms them
-// (fillBCs(r, X.fIndex), field.h:2745-2768): the owner's copy, zero on the
-// field's SYMMETRY patches, the patch value on the tensor diagonal (theta:
-// (value, 0, 0)) on its NEUMANN patches.
-template <typename R>
-__device__ __forceinline__ void ghost_gradient_r(const BcTable& bt, int pi, const R* own, R* out) {
-    const int ku = bt.kind[1][pi], kt = bt.kind[2][pi];
-    const bool zu = ku == BC_SYMMETRY || ku == BC_NEUMANN, zt = kt == BC_SYMMETRY || kt == BC_NEUMANN;
-    for (int c = 0; c < 9; c++) out[c] = zu ? R(0) : own[c];
-    if (ku == BC_NEUMANN) { out[0] = (R)bt.value[1][pi]; out[4] = (R)bt.value[2][pi]; out[8] = (R)bt.value[3][pi]; }
-    for (int c = 9; c < 12; c++) out[c] = zt ? R(0) : own[c];
-    if (kt == BC_NEUMANN) out[9] = (R)bt.value[4][pi];
-}
-
-// Normal components of the viscous fluxes mu grad U (rows 0-2) and
-// mu/Pr grad theta' (row 3) through the area-weighted normal nv.
-template <typename R>
-__device__ __forceinline__ void viscous_normal(const R* g, R mu, R iPr, const R* nv, R* v) {
-    for (int r = 0; r < 3; r++) v[r] = mu * (g[3 * r] * nv[0] + g[3 * r + 1] * nv[1] + g[3 * r + 2] * nv[2]);
-    v[3] = (mu * iPr) * (g[9] * nv[0] + g[10] * nv[1] + g[11] * nv[2]);
-}
-
-// Primitive rows kept in LDS for the face tasks (the owner side of each face
-// node): rho', m (3), Theta', U (3), theta - T0, p'.  c and |U| are
-// recomputed from them with the same operations as make_prim.  The rows are
-// padded by one slot per 8 nodes: a face of constant k reads every 8th node,
-// which would otherwise hit the same few LDS banks.
-constexpr int kPrimRows = 10;
-
-// Work-group of one element (NP threads, one per node; several elements per
-// group when NP < 256).  Phases, each closed by a barrier:
-//   1. own state -> primitives -> contravariant fluxes (15 rows) in LDS;
-//      face tasks issue their neighbour loads
-//   2. volume term along the three GLL lines -> registers
-//   3. own primitives -> LDS (over the flux rows)
-//   4. one thread per face node (6 faces x (N+1)^2 = 384 tasks at N = 7,
-//      one face per wavefront): Rusanov flux -> LDS
-//   5. each node subtracts/adds the fluxes of its faces in face-group order,
-//      then the stage update.
-// AFF: the elements are affine, so the metric is formed from one Jinv and
-// cell volume per element (JcV = Jinv_e (vol_e W), cV = vol_e W with W the
-// node's LGL weight product) instead of being read per node.
-// VISC: artificial viscosity: the flux rows carry -mu grad U and -mu/Pr grad
-// theta' (mu = rho visc) from a.grad, on both sides of every face.
-// MORT: the mesh has 2:1 mortar sides, whose surface terms come from the
-// stage's mortar pre-pass (a separate instantiation, so that conforming
-// meshes run the kernel without the test).
-template <typename R, typename S, int NXc, int NYc, int NZc, bool O32, bool DIN, bool AFF, bool VISC,
-          bool MORT = false>
-__device__ __forceinline__ void rk_stage_body(const DgDev& d, const RkArgs<S>& a) {
-    const int NX = NXc ? NXc : d.npx, NY = NYc ? NYc : d.npy, NZ = NZc ? NZc : d.npz;
-    const int NP = NX * NY * NZ;
-    const int NFN = 2 * (NX * NY + NX * NZ + NY * NZ);
-    // a compile-time shape of more than 128 nodes runs one element per
-    // work-group (the launcher guarantees epb = 1), so the element index is
-    // uniform across the work-group and lives in scalar registers
-    constexpr bool ONE = NXc * NYc * NZc > 128;
-    const int epb = ONE ? 1 : a.epb;
-    const int le = ONE ? 0 : threadIdx.x / NP, q = threadIdx.x - le * NP;
-    // XCD-contiguous element mapping: work-group b runs on XCD b % 8
-    const uint32_t per_xcd = (gridDim.x + 7) / 8;
-    const uint32_t bmap = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    const uint32_t e = bmap * epb + le;
-    const bool active = (ONE ? (int)threadIdx.x < NP : le < epb) && e < d.nelem;
-    extern __shared__ unsigned char lds_raw[];
-    const int per_elem = rk_lds_per_element(NX, NY, NZ);
-    R* G = reinterpret_cast<R*>(lds_raw) + (size_t)le * per_elem;
-    const int NPP = rk_prim_stride(NP);
-    R* FL = G + kPrimRows * NPP;                     // face fluxes [5][NFN]
-    R* Dl = reinterpret_cast<R*>(lds_raw) + (size_t)epb * per_elem;  // D0, D1, D2
-    const int i = q / (NY * NZ), j = (q / NZ) % NY, k = q % NZ;
-    const uint64_t n = (uint64_t)e * NP + q;
-    const uint64_t nb = d.nb;
-    const R T0 = (R)d.T0, gam = (R)d.gamma, gR = (R)(d.gamma * d.R);
-
-    for (int t = threadIdx.x; t < NX * NX + NY * NY + NZ * NZ; t += blockDim.x) {
-        const int s1 = NX * NX, s2 = s1 + NY * NY;
-        Dl[t] = (R)(t < s1 ? d.D[0][t] : t < s2 ? d.D[1][t - s1] : d.D[2][t - s2]);
-    }
-
-
-    Prim<R> P{};
-    // the part of the stage output known before the residual:
-    // b din (+ q on the last stage); the output is pre + b dt L(q + din)
-    double pre[5] = {0, 0, 0, 0, 0};
-    double tpre[5] = {0, 0, 0, 0, 0};  // its tangent (tangent-linear instantiation)
-    R rref = 0, pref = 0, cvn = 1;
-    FaceTask<R> ft{};   // global reads of this thread's first face task
-    constexpr int NG = VISC ? 12 : 1;
-    R gown[NG];          // this node's gradients (VISC)
-    R gA[NG], gB[NG];    // the face task's own-side and far-side gradients (VISC)
-    R rrefA = 0;         // the face task's own-side background density (VISC)
-    const R* grd = static_cast<const R*>(a.grad);
-    if (active) {
-        // all of this phase's global reads first (own node, then the face
-        // task), straight-line, so they are in flight together
-        double base[5], din[5];
-        for (int v = 0; v < 5; v++) {
-            base[v] = ldn<O32>(a.q[v], n);
-            din[v] = ld_delta<O32, DIN>(a.din[v], n);
-        }
-        rref = (R)ldn<O32>(d.rho_ref, n);
-        pref = (R)ldn<O32>(d.p_ref, n);
-        R J[9];
-        if constexpr (AFF) {
-            const double* em = d.emet + (size_t)e * 10;
-            const double cv64 = em[9] * d.wnode[q];
-            cvn = (R)cv64;
-            for (int c = 0; c < 9; c++) J[c] = (R)(em[c] * cv64);
-        } else {
-            if constexpr (sizeof(R) == 4) cvn = ldn<O32>(d.cV32, n);
-            else cvn = (R)ldn<O32>(d.cV, n);
-            if constexpr (sizeof(R) == 4)
-                for (int c = 0; c < 9; c++) J[c] = ldn<O32>(d.JcV32 + (size_t)c * nb, n);
-            else
-                for (int c = 0; c < 9; c++) J[c] = (R)ldn<O32>(d.JcV + (size_t)c * nb, n);
-        }
-        if (q < NFN) prepare_face_task<R, S, O32, DIN>(d, a, e, q, NX, NY, NZ, ft);
-        if constexpr (VISC) {
-            for (int c = 0; c < 12; c++) gown[c] = ldn<O32>(grd + (size_t)c * nb, n);
-            if (q < NFN) {
-                const uint64_t na = (uint64_t)e * NP + ft.fnode;
-                for (int c = 0; c < 12; c++) {
-                    gA[c] = ldn<O32>(grd + (size_t)c * nb, na);
-                    gB[c] = ldn<O32>(grd + (size_t)c * nb, ft.node);
-                }
-                rrefA = (R)ldn<O32>(d.rho_ref, na);
-            }
-        }
-        for (int v = 0; v < 5; v++) {
-            pre[v] = a.last ? base[v] + a.b * din[v] : a.b * din[v];
-            if constexpr (is_dual<R>::value) {
-                const double tb = ldn<O32>(a.tq[v], n), td = ld_delta<O32, DIN>(a.tdin[v], n);
-                tpre[v] = a.last ? tb + a.b * td : a.b * td;
-            }
-        }
-        if constexpr (is_dual<R>::value) {
-            P.rp = load_state<R, S, O32, DIN>(a, 0, n);
-            P.m[0] = load_state<R, S, O32, DIN>(a, 1, n);
-            P.m[1] = load_state<R, S, O32, DIN>(a, 2, n);
-            P.m[2] = load_state<R, S, O32, DIN>(a, 3, n);
-            P.tp = load_state<R, S, O32, DIN>(a, 4, n);
-        } else {
-            P.rp = (R)(base[0] + din[0]);
-            P.m[0] = (R)(base[1] + din[1]); P.m[1] = (R)(base[2] + din[2]); P.m[2] = (R)(base[3] + din[3]);
-            P.tp = (R)(base[4] + din[4]);
-        }
-        make_prim(P, rref, pref, T0, gam, gR, d.ppc);
-        R mu = 0, imu = 0;
-        if constexpr (VISC) {
-            mu = (rref + P.rp) * (R)d.visc;
-            imu = mu * (R)d.iPr;
-        }
-        // rows: rho, m_x, m_y, m_z, Theta
-        for (int row = 0; row < 5; row++) {
-            R f0, f1, f2, g0, g1, g2;
-            flux_row(P, row, T0, f0, f1, f2);
-            if constexpr (VISC) {
-                if (row >= 1 && row <= 3) {
-                    const int r3 = 3 * (row - 1);
-                    f0 = f0 - mu * gown[r3]; f1 = f1 - mu * gown[r3 + 1]; f2 = f2 - mu * gown[r3 + 2];
-                } else if (row == 4) {
-                    f0 = f0 - imu * gown[9]; f1 = f1 - imu * gown[10]; f2 = f2 - imu * gown[11];
-                }
-            }
-            contravariant(J, f0, f1, f2, g0, g1, g2);
-            G[(row * 3 + 0) * NP + q] = g0;
-            G[(row * 3 + 1) * NP + q] = g1;
-            G[(row * 3 + 2) * NP + q] = g2;
-        }
-    }
-    __syncthreads();
-
-    R res[5] = {0, 0, 0, 0, 0};  // volume - surface (= -r of the reference)
-    if (active) {
-        const R* D0 = Dl;
-        const R* D1 = Dl + NX * NX;
-        const R* D2 = D1 + NY * NY;
-        for (int row = 0; row < 5; row++) {
-            const R* G0 = G + (row * 3 + 0) * NP;
-            const R* G1 = G + (row * 3 + 1) * NP;
-            const R* G2 = G + (row * 3 + 2) * NP;
-            R v = 0;
-            for (int t = 0; t < NX; t++) v += D0[t * NX + i] * G0[t * NY * NZ + j * NZ + k];
-            for (int t = 0; t < NY; t++) v += D1[t * NY + j] * G1[i * NY * NZ + t * NZ + k];
-            for (int t = 0; t < NZ; t++) v += D2[t * NZ + k] * G2[i * NY * NZ + j * NZ + t];
-            res[row] = v;
-        }
-    }
-    __syncthreads();
-    if (active) {
-        const R pr[kPrimRows] = {P.rp, P.m[0], P.m[1], P.m[2], P.tp, P.u[0], P.u[1], P.u[2], P.thp, P.pp};
-        for (int r = 0; r < kPrimRows; r++) G[r * NPP + rk_prim_slot(q)] = pr[r];
-    }
-    __syncthreads();
-
-    if (active) {
-        for (int t = q; t < NFN; t += NP) {
-            if (t != q) {
-                prepare_face_task<R, S, O32, DIN>(d, a, e, t, NX, NY, NZ, ft);
-                if constexpr (VISC) {
-                    const uint64_t na = (uint64_t)e * NP + ft.fnode;
-                    for (int c = 0; c < 12; c++) {
-                        gA[c] = ldn<O32>(grd + (size_t)c * nb, na);
-                        gB[c] = ldn<O32>(grd + (size_t)c * nb, ft.node);
-                    }
-                    rrefA = (R)ldn<O32>(d.rho_ref, na);
-                }
-            }
-            const FaceTask<R>& F = ft;
-            if (!((F.meta >> 4) & 1)) continue;
-            if constexpr (MORT)
-                if ((F.meta >> 6) & 1) continue;  // mortar side: surface term from the pre-pass
-            const bool own = (F.meta >> 3) & 1;
-            const bool ghost = (F.meta >> 5) & 1;
-            const int fnode = F.fnode;
-            const R* nv = F.nv;
-            Prim<R> A{};
-            const R* Pf = G + rk_prim_slot(fnode);
-            A.rp = Pf[0 * NPP];
-            A.m[0] = Pf[1 * NPP]; A.m[1] = Pf[2 * NPP]; A.m[2] = Pf[3 * NPP];
-            A.tp = Pf[4 * NPP];
-            A.u[0] = Pf[5 * NPP]; A.u[1] = Pf[6 * NPP]; A.u[2] = Pf[7 * NPP];
-            A.thp = Pf[8 * NPP];
-            A.pp = Pf[9 * NPP];
-            A.c = r_sqrt(gR * (T0 + A.thp));
-            A.umag = r_sqrt(A.u[0] * A.u[0] + A.u[1] * A.u[1] + A.u[2] * A.u[2]);
-            Prim<R> Q{};
-            if (!ghost) {
-                Q.rp = F.rp; Q.m[0] = F.m[0]; Q.m[1] = F.m[1]; Q.m[2] = F.m[2]; Q.tp = F.tp;
-                make_prim(Q, F.rref, F.pref, T0, gam, gR, d.ppc);
-            } else {
-                const BcTable& bt = *d.bc;
-                const int pi = F.meta >> 8;
-                const double uv[3] = {bt.value[1][pi], bt.value[2][pi], bt.value[3][pi]};
-                ghost_state(A, nv, bt.kind[1][pi], uv, F.rref, Q);
-            }
-            R flux[5];
-            if (own) rusanov(A, Q, nv, ghost ? R(0) : R(0.5), T0, flux);
-            else rusanov(Q, A, nv, ghost ? R(0) : R(0.5), T0, flux);
-            if constexpr (VISC) {
-                // central average of -mu grad . n; the far side of a boundary
-                // face takes the ghost gradient and the own density
-                R gG[12];
-                const R* gFar = gB;
-                if (ghost) {
-                    ghost_gradient_r(*d.bc, (int)(F.meta >> 8), gA, gG);
-                    gFar = gG;
-                }
-                const R muA = (rrefA + A.rp) * (R)d.visc;
-                const R muB = ghost ? muA : (F.rref + F.rp) * (R)d.visc;
-                R vA[4], vB[4];
-                viscous_normal(gA, muA, (R)d.iPr, nv, vA);
-                viscous_normal(gFar, muB, (R)d.iPr, nv, vB);
-                const R fI = ghost ? R(0) : R(0.5), fJ = R(1) - fI;
-                const R* vO = own ? vA : vB;
-                const R* vN = own ? vB : vA;
-                for (int r = 0; r < 4; r++) flux[1 + r] = flux[1 + r] - (vO[r] * fI + vN[r] * fJ);
-            }
-            for (int v = 0; v < 5; v++) FL[v * NFN + t] = flux[v];
-        }
-    }
-    __syncthreads();
-    if (!active) return;
-
-    for (int g = 0; g < 6; g++) {
-        if (!on_face(g, i, j, k, NX, NY, NZ)) continue;
-        const uint32_t meta = d.eface[(size_t)e * 6 + g].meta;
-        if (!((meta >> 4) & 1)) continue;
-        int fa, fb;
-        face_ab(g, i, j, k, fa, fb);
-        if constexpr (MORT) {
-            if ((meta >> 6) & 1) {
-                // 2:1 mortar side: its surface term, sign included, from the
-                // stage's mortar pre-pass
-                const size_t mi = ((size_t)(meta >> 8) * d.npfm + fa * (g < 2 ? NY : NZ) + fb) * 5;
-                for (int v = 0; v < 5; v++) {
-                    R x = (R)d.msurf[mi + v];
-                    if constexpr (is_dual<R>::value) x.d[0] = d.msurf_t[mi + v];
-                    res[v] += x;
-                }
-                continue;
-            }
-        }
-        const int t = face_task_index(g, fa, fb, NX, NY, NZ);
-        if ((meta >> 3) & 1)
-            for (int v = 0; v < 5; v++) res[v] -= FL[v * NFN + t];
-        else
-            for (int v = 0; v < 5; v++) res[v] += FL[v * NFN + t];
-    }
-    // L(q) = (volume - surface)/cV + buoyancy; increments and base
-    const R icv = r_div(R(1), cvn);
-    R Lq[5];
-    for (int v = 0; v < 5; v++) Lq[v] = res[v] * icv;
-    if (d.buoyancy) {
-        Lq[1] += P.rp * (R)d.g[0];
-        Lq[2] += P.rp * (R)d.g[1];
-        Lq[3] += P.rp * (R)d.g[2];
-    }
-    for (int v = 0; v < 5; v++) {
-        const double out = pre[v] + a.bdt * value_of(Lq[v]);
-        if (a.last) stn<O32>(a.qout[v], n, out);
-        else stn<O32>(a.dout[v], n, (S)out);
-        if constexpr (is_dual<R>::value) {
-            const double tout = tpre[v] + a.bdt * Lq[v].d[0];
-            if (a.last) stn<O32>(a.tqout[v], n, tout);
-            else stn<O32>(a.tdout[v], n, tout);
-        }
-    }
-    if (a.check) {
-        bool bad = false;
-        for (int v = 0; v < 5; v++) bad |= !isfinite(value_of(Lq[v]));
-        if (bad) *a.flag = 1;
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Strong gradients of U and theta' at the stage state Q = q + din of the
@@ -717,100 +295,6 @@ template hipError_t launch_mol_gradient<double, double>(const DgDev&, const doub
 template hipError_t launch_mol_gradient<float, float>(const DgDev&, const double* const[5], const float* const[5],
                                                       float*, hipStream_t);
 
-template <typename R, typename S, int X, int Y, int Z, bool DIN, bool AFF, bool VISC, bool MORT = false>
-__global__ void __launch_bounds__(512) rk_stage_kernel(DgDev d, RkArgs<S> a) {
-    rk_stage_body<R, S, X, Y, Z, false, DIN, AFF, VISC, MORT>(d, a);
-}
-
-// Compile-time element shape (X x Y x Z nodes), node offsets in 32 bits,
-// registers capped at W waves per SIMD.  Measured on the 64x64x32 N=7
-// workload, FP32 runs fastest at 6 (three work-groups per CU) and FP64 at 4
-// (two work-groups per CU).  Shapes of up to 128 nodes hold several elements
-// per work-group, whose element index is not uniform and costs registers, so
-// they take one wave less (FP64 at 4^3 nodes two less: at 3 waves it spills
-// 56 bytes per lane and ran 8% slower than at 2); the viscous variant's extra
-// gradient state takes two less.  FP32 at 6^3 nodes (N = 5) spills a few
-// dwords at 6 and runs 5-6% faster at 5.  Measured and not taken: FP32 4^3
-// at 4 (2% slower than 5), FP64 5^3 at 2 (18% slower than 3).
-template <typename R, int X, int Y, int Z, bool VISC>
-constexpr int rk_waves_per_simd() {
-    constexpr int np = X * Y * Z;
-    if constexpr (sizeof(R) == 4) return VISC ? 4 : (np > 128 ? (np == 216 ? 5 : 6) : 5);
-    return VISC ? 2 : (np > 128 ? 4 : np > 64 ? 3 : 2);
-}
-
-template <typename R, typename S, int X, int Y, int Z, int W, bool DIN, bool AFF, bool VISC, bool MORT = false>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(W)))
-rk_stage_kernel_fx(DgDev d, RkArgs<S> a) {
-    rk_stage_body<R, S, X, Y, Z, true, DIN, AFF, VISC, MORT>(d, a);
-}
-
-template <typename R, typename S, int X, int Y, int Z, bool DIN, bool AFF, bool VISC, bool MORT = false>
-static void launch_rk_kernel(const DgDev& d, const RkArgs<S>& a, unsigned blocks, int threads, size_t lds,
-                             hipStream_t st) {
-    constexpr int W = rk_waves_per_simd<R, X, Y, Z, VISC>();
-    if constexpr (X > 0 && !is_dual<R>::value) {
-        if (d.nb * sizeof(double) < (1ull << 32)) {
-            hipLaunchKernelGGL((rk_stage_kernel_fx<R, S, X, Y, Z, W, DIN, AFF, VISC, MORT>), dim3(blocks),
-                               dim3(threads), lds, st, d, a);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((rk_stage_kernel<R, S, X, Y, Z, DIN, AFF, VISC, MORT>), dim3(blocks), dim3(threads), lds, st,
-                       d, a);
-}
-
-template <typename R, typename S, int X, int Y, int Z, bool DIN>
-static void launch_rk_metric(const DgDev& d, const RkArgs<S>& a, unsigned blocks, int threads, size_t lds,
-                             hipStream_t st) {
-    // the tangent-linear instantiation has no viscous variant (the
-    // derivative entry points refuse diffusion)
-    {
-        // 2:1 non-conforming meshes (inviscid)
-        if (d.nmort) {
-            if constexpr (!is_dual<R>::value) {
-                if (a.grad) {
-                    if (d.affine) launch_rk_kernel<R, S, X, Y, Z, DIN, true, true, true>(d, a, blocks, threads, lds, st);
-                    else launch_rk_kernel<R, S, X, Y, Z, DIN, false, true, true>(d, a, blocks, threads, lds, st);
-                    return;
-                }
-            }
-            if (d.affine) launch_rk_kernel<R, S, X, Y, Z, DIN, true, false, true>(d, a, blocks, threads, lds, st);
-            else launch_rk_kernel<R, S, X, Y, Z, DIN, false, false, true>(d, a, blocks, threads, lds, st);
-            return;
-        }
-    }
-    if constexpr (!is_dual<R>::value) {
-        if (a.grad) {
-            if (d.affine) launch_rk_kernel<R, S, X, Y, Z, DIN, true, true>(d, a, blocks, threads, lds, st);
-            else launch_rk_kernel<R, S, X, Y, Z, DIN, false, true>(d, a, blocks, threads, lds, st);
-            return;
-        }
-    }
-    if (d.affine) launch_rk_kernel<R, S, X, Y, Z, DIN, true, false>(d, a, blocks, threads, lds, st);
-    else launch_rk_kernel<R, S, X, Y, Z, DIN, false, false>(d, a, blocks, threads, lds, st);
-}
-
-template <typename R, typename S, int X, int Y, int Z>
-static hipError_t launch_rk_t(const DgDev& d, const RkArgs<S>& a_in, hipStream_t st) {
-    RkArgs<S> a = a_in;
-    const int NP = d.np;
-    if (NP > 512) return hipErrorInvalidValue;
-    // elements per work-group: fill 256 threads, as far as the LDS allows
-    int epb = NP >= 256 ? 1 : 256 / NP;
-    while (epb > 1 && rk_lds_bytes(d.npx, d.npy, d.npz, epb, sizeof(R)) > 65536) epb--;
-    int threads = (epb * NP + 63) / 64 * 64;
-    unsigned blocks = (d.nelem + epb - 1) / epb;
-    blocks = (blocks + 7) / 8 * 8;  // whole XCD chunks
-    const size_t lds = rk_lds_bytes(d.npx, d.npy, d.npz, epb, sizeof(R));
-    if (lds > 65536) return hipErrorInvalidValue;
-    if (X * Y * Z > 128 && epb != 1) return hipErrorInvalidValue;  // the body assumes one element
-    a.epb = epb;
-    if (a.din[0]) launch_rk_metric<R, S, X, Y, Z, true>(d, a, blocks, threads, lds, st);
-    else launch_rk_metric<R, S, X, Y, Z, false>(d, a, blocks, threads, lds, st);
-    return hipGetLastError();
-}
-
 // ---------------------------------------------------------------------------
 // 2:1 non-conforming faces of the method-of-lines stage (field.h:2018-2248,
 // 2927-2943, 3085-3117).  On a mortar face the coarse side's node values
@@ -977,6 +461,8 @@ hipError_t launch_rk_shape(const DgDev& d, const RkArgs<S>& a, hipStream_t st) {
     if (d.npx == 5 && d.npy == 5 && d.npz == 5) return launch_rk_t<R, S, 5, 5, 5>(d, a, st);
     if (d.npx == 4 && d.npy == 4 && d.npz == 4) return launch_rk_t<R, S, 4, 4, 4>(d, a, st);
     if (d.npx == 5 && d.npy == 1 && d.npz == 5) return launch_rk_t<R, S, 5, 1, 5>(d, a, st);
+    if (d.npx == 6 && d.npy == 1 && d.npz == 6) return launch_rk_t<R, S, 6, 1, 6>(d, a, st);
+    if (d.npx == 7 && d.npy == 1 && d.npz == 7) return launch_rk_t<R, S, 7, 1, 7>(d, a, st);
     return launch_rk_t<R, S, 0, 0, 0>(d, a, st);
 }
 

@@ -1,0 +1,778 @@
+// Method-of-lines dGSEM Euler residual fused with an SSP-RK3 stage
+// (Shu-Osher form, written as increments over the step's base state):
+//
+//   d1 = dt L(q)            d2 = (d1 + dt L(q + d1)) / 4
+//   d3 = 2 (d2 + dt L(q + d2)) / 3                  q^{n+1} = q + d3
+//
+// State: conserved perturbations over the FP64 hydrostatic background,
+//   rho' = rho - rho_ref,  m = rho U,  Theta' = rho theta - rho_ref T0.
+// Spatial operator: the reference's (divf + rusanov + div_flux + src,
+// field.h:2927-2943, 3085-3117, 3416-3478, 3711-3723) with all fluxes
+// evaluated at one state: F_rho = m, F_m = m (x) U + p' I, F_Theta = m theta,
+// lambda = (avg|U| + avg sqrt(gamma R theta)) / 2, normal-only momentum
+// dissipation, buoyancy (rho - rho_ref) g.  p' = p_ref expm1(gamma
+// log1p(Theta'/(rho_ref T0))) is the exact p(rho theta) - p_ref without the
+// cancellation, so the flux never touches the background's hydrostatic
+// balance.
+//
+// Template parameters: R the arithmetic type of the residual (double, or
+// float for the FP32-perturbation form), S the storage type of the stage
+// increments.  The base state and the final accumulation q + d3 are FP64 in
+// both forms; the background is FP64 and converted once per node.
+//
+// One work-group per element (NP threads, NP = 512 at N = 7; several elements
+// of the smaller shapes): contravariant fluxes of the 5 equations staged in
+// LDS (15 x NP values), transposed 1-D derivative along the three GLL lines,
+// Rusanov surface terms from the neighbour traces (global, L2/MALL resident),
+// update fused.  Work-groups are mapped to elements XCD-contiguously so face
+// neighbours share an L2.
+//
+// The kernel is bound by instruction issue (the vector ALU is busy in about
+// two cycles of three; memory moves at half of a copy's rate), so it is
+// written for few instructions and no waits between them:
+//  - face terms in the outward normal, one sequence of code for either side
+//    of a face; the element faces' normals and scales come from a table in
+//    the residual's type, and on affine elements the FP64 form's weights
+//    cancel against the mass matrix, so no weight or volume is read per node;
+//  - reciprocals and roots by Newton steps instead of the IEEE sequences;
+//  - face tasks are dealt over the whole work-group (not a wave per face), the
+//    neighbours' traces are loaded before the volume term and first of all
+//    loads, since loads return in order; lanes without a node repeat the
+//    last one, so no load sits behind a branch;
+//  - 2D decks without y faces skip that direction at compile time; meshes too
+//    small to fill the chip take fewer elements per work-group.
+// Measured before and after (stages of 16^3 elements and up, G node.stages/s
+// x 5): N = 7 FP64 111 -> 131, FP32 175 -> 166; N = 3 FP32 107 -> 143; N = 4
+// FP64 68 -> 113; the 2D N = 4 deck of 62,500 nodes 31 -> 21 us a step.
+//
+// The method-of-lines path has no bit-level counterpart in the reference, so
+// products and sums are fused into FMAs here, in the headers' inline physics
+// too (the split reference-order kernels keep the build-wide
+// -ffp-contract=off).
+#pragma once
+#pragma clang fp contract(fast)
+
+#include "dg_kernels.hpp"
+#include "dg_physics.hpp"
+
+namespace nsem {
+
+namespace {
+
+// Stores of the stage output bypass the caches' retention (non-temporal):
+// they are not read again in this launch, and the L2 keeps the neighbour
+// traces instead.
+template <bool O32, typename T>
+__device__ __forceinline__ void stn(T* base, uint64_t i, T v) {
+    if constexpr (O32)
+        __builtin_nontemporal_store(v, reinterpret_cast<T*>(reinterpret_cast<char*>(base) + byte_off(i, sizeof(T))));
+    else
+        __builtin_nontemporal_store(v, base + i);
+}
+
+// Increment of variable v at node n (DIN: the stage has one; a compile-time
+// choice, so the loads carry no null-pointer branches between them).
+template <bool O32, bool DIN, typename S>
+__device__ __forceinline__ double ld_delta(const S* d, uint64_t i) {
+    if constexpr (DIN) return (double)ldn<O32>(d, i);
+    else return 0.0;
+}
+
+// State q + d_in of variable v at node n in the residual type (with its
+// tangent for the tangent-linear instantiation).
+template <typename R, typename S, bool O32, bool DIN>
+__device__ __forceinline__ R load_state(const RkArgs<S>& a, int v, uint64_t n) {
+    const double x = ldn<O32>(a.q[v], n) + ld_delta<O32, DIN>(a.din[v], n);
+    if constexpr (is_dual<R>::value) {
+        R r(x);
+        r.d[0] = ldn<O32>(a.tq[v], n) + ld_delta<O32, DIN>(a.tdin[v], n);
+        return r;
+    } else {
+        return (R)x;
+    }
+}
+
+}  // namespace
+
+// The coefficients of the equation of state's series in the residual type.
+template <typename R>
+__device__ __forceinline__ const auto* series(const DgDev& d) {
+    if constexpr (sizeof(R) == 4) return d.ppc32;
+    else return d.ppc;
+}
+// The hydrostatic background at a node in the residual type (the FP32 copies
+// hold the FP64 values rounded, as the FP32 form uses them).
+template <typename R, bool O32>
+__device__ __forceinline__ void load_background(const DgDev& d, uint64_t n, R& rref, R& pref) {
+    if constexpr (sizeof(R) == 4) {
+        rref = ldn<O32>(d.rho_ref32, n);
+        pref = ldn<O32>(d.p_ref32, n);
+    } else {
+        rref = (R)ldn<O32>(d.rho_ref, n);
+        pref = (R)ldn<O32>(d.p_ref, n);
+    }
+}
+
+// What a face needs of the state on one of its sides: rho', m, Theta', 1/rho,
+// theta - T0, p' and |U| + c.
+template <typename R>
+struct Trace {
+    R rp, m[3], tp, ir, thp, pp, cu;
+};
+
+template <typename R>
+__device__ __forceinline__ R speed_plus_c(const R* m, R ir, R thp, R T0, R gR) {
+    return r_root(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]) * ir + r_root(gR * (T0 + thp));
+}
+
+// Everything but cu from rp, m, tp.
+template <typename R>
+__device__ __forceinline__ void complete(Trace<R>& t, R rref, R pref, R T0, R gam, const DgDev& d) {
+    t.ir = r_rcp(rref + t.rp);
+    t.thp = (t.tp - T0 * t.rp) * t.ir;
+    t.pp = pref * pow1p_m1(t.tp * r_rcp(rref * T0), gam, series<R>(d));
+}
+
+// Everything one face-node task reads from global memory, gathered before
+// the volume term so that its latency overlaps the element's own loads:
+// the face entry, the outward unit normal with its scale and the neighbour's
+// state (on a boundary or absent face the element's own face node is read
+// instead, so the loads need no branch).  The two nodes of a conforming face
+// lie at one point, so the far side takes the near side's background.
+template <typename R>
+struct FaceTask {
+    uint32_t meta;
+    uint64_t node;    // the node the state was read from (neighbour, or own on a boundary)
+    R en[3], s;
+    R rp, m[3], tp;
+};
+
+// Face-node tasks of an element; YF: false when no y face of the mesh is
+// present (the 2D decks: one element in y of order 0), so that groups 2 and 3
+// have no tasks.
+template <bool YF>
+__host__ __device__ constexpr int rk_face_nodes(int NX, int NY, int NZ) {
+    return 2 * (NX * NY + (YF ? NX * NZ : 0) + NY * NZ);
+}
+
+// The first step of a face-node task: its face entry's other element and meta
+// word, on which the addresses of its other reads depend.
+struct FaceEntry {
+    uint32_t other, meta;
+};
+
+template <bool YF>
+__device__ __forceinline__ void locate_face_task(int t, int NX, int NY, int NZ, int& g, int& fa, int& fb, int& fnode) {
+    if constexpr (!YF) t += t < 2 * NX * NY ? 0 : 2 * NX * NZ;
+    face_task(t, NX, NY, NZ, g, fa, fb, fnode);
+}
+
+template <bool YF>
+__device__ __forceinline__ FaceEntry load_face_entry(const DgDev& d, uint32_t e, int t, int NX, int NY, int NZ) {
+    int g, fa, fb, fnode;
+    locate_face_task<YF>(t, NX, NY, NZ, g, fa, fb, fnode);
+    const EFace* f = d.eface + (e * 6 + g);
+    return FaceEntry{f->other, f->meta};
+}
+
+template <typename R, typename S, bool O32, bool DIN, bool YF>
+__device__ __forceinline__ void prepare_face_task(const DgDev& d, const RkArgs<S>& a, uint32_t e, int t,
+                                                  const FaceEntry& fe, int NX, int NY, int NZ, FaceTask<R>& F) {
+    int g, fa, fb, fnode;
+    locate_face_task<YF>(t, NX, NY, NZ, g, fa, fb, fnode);
+    F.meta = fe.meta;
+    const bool interior = (fe.meta & 0x30) == 0x10;   // present, no ghost
+    // (selects, not a branch: a branch would wait for the entry twice)
+    const uint64_t m = face_node(interior ? fe.other : e, interior ? (int)(fe.meta & 7) : g, fa, fb, NX, NY, NZ);
+    F.node = m;
+    F.rp = load_state<R, S, O32, DIN>(a, 0, m);
+    F.m[0] = load_state<R, S, O32, DIN>(a, 1, m);
+    F.m[1] = load_state<R, S, O32, DIN>(a, 2, m);
+    F.m[2] = load_state<R, S, O32, DIN>(a, 3, m);
+    F.tp = load_state<R, S, O32, DIN>(a, 4, m);
+}
+
+// The task's outward unit normal and scale (read after the volume term, when
+// registers are free again).
+template <typename R, bool AFF, bool YF>
+__device__ __forceinline__ void load_face_normal(const DgDev& d, uint32_t e, int t, int NX, int NY, int NZ,
+                                                 FaceTask<R>& F) {
+    int g, fa, fb, fnode;
+    locate_face_task<YF>(t, NX, NY, NZ, g, fa, fb, fnode);
+    const uint32_t ef6 = e * 6 + g;
+    if constexpr (sizeof(R) == 4) {
+        const float4 fn = reinterpret_cast<const float4*>(d.fnorm32)[ef6];
+        F.en[0] = fn.x; F.en[1] = fn.y; F.en[2] = fn.z; F.s = fn.w;
+    } else {
+        const double* fn = d.fnorm + (size_t)ef6 * 4;
+        F.en[0] = (R)fn[0]; F.en[1] = (R)fn[1]; F.en[2] = (R)fn[2]; F.s = (R)fn[3];
+    }
+    if constexpr (!AFF) {
+        // the face-node weight w_a w_b / 4
+        const double* wa = g < 4 ? d.w[0] : d.w[1];
+        const double* wb = g < 2 ? d.w[1] : d.w[2];
+        F.s = F.s * (R)(wa[fa] * wb[fb] / 4);
+    }
+}
+
+// SYMMETRY ghost of a vector through the unit normal e (as sym_r).
+template <typename R>
+__device__ __forceinline__ void sym_unit(const R* p, const R* e, R* r) {
+    const R dn = e[0] * p[0] + e[1] * p[1] + e[2] * p[2];
+    r[0] = p[0] - e[0] * dn; r[1] = p[1] - e[1] * dn; r[2] = p[2] - e[2] * dn;
+    const R mr = r_sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
+    if (mr <= R(1e-7)) return;
+    const R s = r_div(r_sqrt(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]), mr);
+    r[0] *= s; r[1] *= s; r[2] *= s;
+}
+
+// Ghost side of a boundary face from the element's side A (as ghost_state):
+// momentum by the velocity condition, scalars copied.  The SYMMETRY ghost of
+// the velocity and of the momentum are each rescaled to their own length.
+template <typename R>
+__device__ __forceinline__ void ghost_trace(const Trace<R>& A, const R* en, int kind, const double* uval, R rref,
+                                            R T0, R gR, Trace<R>& Q, R& unQ) {
+    Q = A;
+    R u[3] = {A.m[0] * A.ir, A.m[1] * A.ir, A.m[2] * A.ir};
+    if (kind == BC_SYMMETRY) {
+        R v[3];
+        sym_unit(u, en, v);
+        for (int c = 0; c < 3; c++) u[c] = v[c];
+        sym_unit(A.m, en, Q.m);
+    } else if (kind == BC_DIRICHLET) {
+        const R rho = rref + A.rp;
+        for (int c = 0; c < 3; c++) {
+            u[c] = R(uval[c]);
+            Q.m[c] = rho * u[c];
+        }
+    }
+    unQ = u[0] * en[0] + u[1] * en[1] + u[2] * en[2];
+    Q.cu = r_sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]) + r_sqrt(gR * (T0 + A.thp));
+}
+
+// Rusanov flux through the outward unit normal en from the element's side A to
+// the far side Q (field.h:2927-2943), the same number from either side: the
+// averages are symmetric and the jumps change sign with the normal.  L: the
+// state averaged with Q, A inside, Q itself on a boundary (where the flux
+// takes the ghost's values).
+template <typename R>
+__device__ __forceinline__ void rusanov_out(const Trace<R>& A, const Trace<R>& L, const Trace<R>& Q, R mnA, R mnL,
+                                            R mnQ, R unL, R unQ, const R* en, R T0, R f[5]) {
+    const R lam = (L.cu + Q.cu) * R(0.25), hL = unL * R(0.5), hQ = unQ * R(0.5);
+    f[0] = (mnL + mnQ) * R(0.5) - lam * (Q.rp - A.rp);
+    const R pn = (L.pp + Q.pp) * R(0.5) - lam * (mnQ - mnA);
+    for (int r = 0; r < 3; r++) f[1 + r] = L.m[r] * hL + Q.m[r] * hQ + pn * en[r];
+    f[4] = ((mnL * T0 + mnL * L.thp) + (mnQ * T0 + mnQ * Q.thp)) * R(0.5) - lam * (Q.tp - A.tp);
+}
+
+// Ghost-node gradients of the viscous terms, as the split step forms them
+// (fillBCs(r, X.fIndex), field.h:2745-2768): the owner's copy, zero on the
+// field's SYMMETRY patches, the patch value on the tensor diagonal (theta:
+// (value, 0, 0)) on its NEUMANN patches.
+template <typename R>
+__device__ __forceinline__ void ghost_gradient_r(const BcTable& bt, int pi, const R* own, R* out) {
+    const int ku = bt.kind[1][pi], kt = bt.kind[2][pi];
+    const bool zu = ku == BC_SYMMETRY || ku == BC_NEUMANN, zt = kt == BC_SYMMETRY || kt == BC_NEUMANN;
+    for (int c = 0; c < 9; c++) out[c] = zu ? R(0) : own[c];
+    if (ku == BC_NEUMANN) { out[0] = (R)bt.value[1][pi]; out[4] = (R)bt.value[2][pi]; out[8] = (R)bt.value[3][pi]; }
+    for (int c = 9; c < 12; c++) out[c] = zt ? R(0) : own[c];
+    if (kt == BC_NEUMANN) out[9] = (R)bt.value[4][pi];
+}
+
+// Normal components of the viscous fluxes mu grad U (rows 0-2) and
+// mu/Pr grad theta' (row 3) through the area-weighted normal nv.
+template <typename R>
+__device__ __forceinline__ void viscous_normal(const R* g, R mu, R iPr, const R* nv, R* v) {
+    for (int r = 0; r < 3; r++) v[r] = mu * (g[3 * r] * nv[0] + g[3 * r + 1] * nv[1] + g[3 * r + 2] * nv[2]);
+    v[3] = (mu * iPr) * (g[9] * nv[0] + g[10] * nv[1] + g[11] * nv[2]);
+}
+
+// Form the value at this point of the program (the volume sums would
+// otherwise be sunk past the barriers to their use, with every operand kept).
+template <typename R>
+__device__ __forceinline__ void keep_here(R& v) {
+    if constexpr (is_dual<R>::value) __asm__ volatile("" : "+v"(v.v), "+v"(v.d[0]));
+    else __asm__ volatile("" : "+v"(v));
+}
+
+// Trace rows kept in LDS for the face tasks (the element's side of each face
+// node): rho', m (3), Theta', 1/rho, theta - T0, p', rho_ref, p_ref; |U| + c is
+// formed from them where it is used.  The rows are padded by one slot per 8 nodes: a face
+// of constant k reads every 8th node, which would otherwise hit the same few
+// LDS banks.
+constexpr int kTraceRows = 10;
+
+// Work-group of one element (NP threads, one per node; several elements per
+// group when NP <= 128).  Phases, each closed by a barrier:
+//   1. own state -> contravariant fluxes (15 rows) in LDS; face tasks issue
+//      their neighbour loads
+//   2. volume term along the three GLL lines -> registers
+//   3. own traces -> LDS (over the flux rows)
+//   4. one thread per face node (6 faces x (N+1)^2 = 384 tasks at N = 7,
+//      one face per wavefront): outward Rusanov flux -> LDS
+//   5. each node subtracts the fluxes of its faces in face-group order, then
+//      the stage update.
+// What bounds it: the VALU issue slots, two thirds busy with 734 instructions
+// a wave at N = 7 and 1,155 at N = 3 in an earlier form of this kernel, the
+// rest waiting for memory.  So the arithmetic is what was cut:
+//   - threads without a node repeat the last one and only their stores are
+//     held back (the branches' zero-filled registers were 100 moves);
+//   - the flux is formed through the outward normal, so owner and neighbour,
+//     often both in one wave, run the same instructions;
+//   - unit normals and their scales come from a table, not from a square root
+//     and a division per face node;
+//   - reciprocals and roots are a Newton step on the hardware's approximation
+//     instead of the IEEE sequences (r_rcp, r_root);
+//   - on affine elements (AFF) the node weights cancel: JcV = Jinv vol W and
+//     cV = vol W with W the node's LGL weights, so the volume term is
+//     M_d Jinv F with M_d[t][i] = D_d[t][i] w_t / w_i (d.DWm), and a face's
+//     scale is |facet| 2 / vol, times 1 / w_end where it is subtracted; no metric or volume per node is formed
+//     and nothing is divided by cV.
+// The face tasks are dealt out over the whole group: at 4^3 nodes 384 tasks
+// of four elements fill six of the eight wave passes that 96 per element took.
+// VISC: artificial viscosity: the flux rows carry -mu grad U and -mu/Pr grad
+// theta' (mu = rho visc) from a.grad, on both sides of every face.
+// MORT: the mesh has 2:1 mortar sides, whose surface terms come from the
+// stage's mortar pre-pass (a separate instantiation, so that conforming
+// meshes run the kernel without the test).
+template <typename R, typename S, int NXc, int NYc, int NZc, bool O32, bool DIN, bool AFF, bool VISC, bool MORT,
+          bool YF>
+__device__ __forceinline__ void rk_stage_body(const DgDev& d, const RkArgs<S>& a) {
+    const int NX = NXc ? NXc : d.npx, NY = NYc ? NYc : d.npy, NZ = NZc ? NZc : d.npz;
+    const int NP = NX * NY * NZ;
+    const int NFN = rk_face_nodes<YF>(NX, NY, NZ);
+    // a compile-time shape of more than 128 nodes runs one element per
+    // work-group (the launcher guarantees epb = 1), so the element index is
+    // uniform across the work-group and lives in scalar registers
+    constexpr int NPc = NXc * NYc * NZc;
+    constexpr bool ONE = NPc > 128;
+    constexpr bool YL = NYc != 1;   // a y line has a derivative
+    const int epb = ONE ? 1 : a.epb;
+    // XCD-contiguous element mapping: work-group b runs on XCD b % 8
+    const uint32_t per_xcd = (gridDim.x + 7) / 8;
+    const uint32_t bmap = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    const uint32_t e0 = bmap * epb;
+    if (e0 >= d.nelem) return;
+    const int tid = threadIdx.x;
+    const int le = ONE ? 0 : min(tid / NP, epb - 1);
+    const int q = ONE && NPc % 64 == 0 ? tid : min(tid - le * NP, NP - 1);
+    const uint32_t e = ONE ? e0 : min(e0 + le, d.nelem - 1);
+    const bool active = (ONE && NPc % 64 == 0) || (tid < epb * NP && (ONE || e0 + le < d.nelem));
+    extern __shared__ unsigned char lds_raw[];
+    const int per_elem = rk_lds_per_element(NX, NY, NZ);
+    R* LDS = reinterpret_cast<R*>(lds_raw);
+    R* G = LDS + le * per_elem;
+    const int NPP = rk_prim_stride(NP);
+    R* Dl = LDS + epb * per_elem;  // the three derivative matrices
+    const int i = q / (NY * NZ), j = (q / NZ) % NY, k = q % NZ;
+    const uint64_t n = (uint64_t)e * NP + q;
+    const uint64_t nb = d.nb;
+    const R T0 = (R)d.T0, gam = (R)d.gamma, gR = (R)(d.gamma * d.R);
+    const int threads = ONE ? (NPc + 63) / 64 * 64 : (epb * NP + 63) / 64 * 64;
+    const int nD = NX * NX + NY * NY + NZ * NZ;
+    auto Dat = [&](int t) -> R {
+        if constexpr (sizeof(R) == 4) return d.Dm32[t];
+        else return (R)(AFF ? d.DWm : d.Dm)[t];
+    };
+    // (the first entry of each thread; a 2D group has fewer threads than entries)
+    const R D1st = Dat(min(tid, nD - 1));
+    // face tasks of the group: task tid + p threads in pass p; the first PF
+    // passes' loads are issued with the node's own
+    const int tasks = epb * NFN;
+    const int wave0 = __builtin_amdgcn_readfirstlane(tid);
+    constexpr int PF = VISC || is_dual<R>::value || !NPc ? 1 : rk_face_nodes<YF>(NXc, NYc, NZc) > NPc ? 2 : 1;
+    FaceTask<R> ft[PF];
+    auto task_of = [&](int t, int& lt, int& tl) {
+        t = min(t, tasks - 1);
+        lt = ONE ? 0 : t / NFN;
+        tl = t - lt * NFN;
+    };
+    auto entry = [&](int t) {
+        int lt, tl;
+        task_of(t, lt, tl);
+        return load_face_entry<YF>(d, ONE ? e0 : min(e0 + lt, d.nelem - 1), tl, NX, NY, NZ);
+    };
+    auto prepare = [&](int t, const FaceEntry& fe, FaceTask<R>& F) {
+        int lt, tl;
+        task_of(t, lt, tl);
+        prepare_face_task<R, S, O32, DIN, YF>(d, a, ONE ? e0 : min(e0 + lt, d.nelem - 1), tl, fe, NX, NY, NZ, F);
+    };
+    auto normal = [&](int t, FaceTask<R>& F) {
+        int lt, tl;
+        task_of(t, lt, tl);
+        load_face_normal<R, AFF, YF>(d, ONE ? e0 : min(e0 + lt, d.nelem - 1), tl, NX, NY, NZ, F);
+    };
+    // The order of the reads: loads return in order, so what a wait is for
+    // comes first.  The face entries, whose tasks' addresses wait for them,
+    // then the node's own state, then the tasks' reads while that is under way.
+    FaceEntry fe[PF];
+#pragma unroll
+    for (int p = 0; p < PF; p++) fe[p] = entry(tid + p * threads);
+    __builtin_amdgcn_sched_barrier(0);
+
+    Trace<R> A;
+    // the part of the stage output known before the residual:
+    // b din (+ q on the last stage); the output is pre + b dt L(q + din)
+    double pre[5];
+    double tpre[5];  // its tangent (tangent-linear instantiation)
+    R rref, pref, cvn = 1;
+    constexpr int NG = VISC ? 12 : 1;
+    R gown[NG];          // this node's gradients (VISC)
+    const R* grd = static_cast<const R*>(a.grad);
+    {
+        double base[5], din[5];
+        for (int v = 0; v < 5; v++) {
+            base[v] = ldn<O32>(a.q[v], n);
+            din[v] = ld_delta<O32, DIN>(a.din[v], n);
+        }
+        load_background<R, O32>(d, n, rref, pref);
+        R J[9];
+        if constexpr (AFF) {
+            for (int c = 0; c < 9; c++) J[c] = (R)d.emet[(size_t)e * 10 + c];
+        } else {
+            if constexpr (sizeof(R) == 4) cvn = ldn<O32>(d.cV32, n);
+            else cvn = (R)ldn<O32>(d.cV, n);
+            if constexpr (sizeof(R) == 4)
+                for (int c = 0; c < 9; c++) J[c] = ldn<O32>(d.JcV32 + (size_t)c * nb, n);
+            else
+                for (int c = 0; c < 9; c++) J[c] = (R)ldn<O32>(d.JcV + (size_t)c * nb, n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = 0; p < PF; p++)
+            if (wave0 + p * threads < tasks) prepare(tid + p * threads, fe[p], ft[p]);
+        if (tid < nD) Dl[tid] = D1st;
+        if constexpr (!NPc || NXc * NXc + NYc * NYc + NZc * NZc > (NPc + 63) / 64 * 64)
+            for (int t = tid + threads; t < nD; t += threads) Dl[t] = Dat(t);
+        if constexpr (VISC)
+            for (int c = 0; c < 12; c++) gown[c] = ldn<O32>(grd + (size_t)c * nb, n);
+        for (int v = 0; v < 5; v++) {
+            pre[v] = a.last ? base[v] + a.b * din[v] : a.b * din[v];
+            if constexpr (is_dual<R>::value) {
+                const double tb = ldn<O32>(a.tq[v], n), td = ld_delta<O32, DIN>(a.tdin[v], n);
+                tpre[v] = a.last ? tb + a.b * td : a.b * td;
+            }
+        }
+        if constexpr (is_dual<R>::value) {
+            A.rp = load_state<R, S, O32, DIN>(a, 0, n);
+            for (int c = 0; c < 3; c++) A.m[c] = load_state<R, S, O32, DIN>(a, 1 + c, n);
+            A.tp = load_state<R, S, O32, DIN>(a, 4, n);
+        } else {
+            A.rp = (R)(base[0] + din[0]);
+            for (int c = 0; c < 3; c++) A.m[c] = (R)(base[1 + c] + din[1 + c]);
+            A.tp = (R)(base[4] + din[4]);
+        }
+        // base and din end here (their last uses would otherwise be put off
+        // past the equation of state, which needs their registers)
+        for (int v = 0; v < 5; v++) __asm__ volatile("" : "+v"(pre[v]));
+        complete(A, rref, pref, T0, gam, d);
+        const R u[3] = {A.m[0] * A.ir, A.m[1] * A.ir, A.m[2] * A.ir};
+        R mu = 0, imu = 0;
+        if constexpr (VISC) {
+            mu = (rref + A.rp) * (R)d.visc;
+            imu = mu * (R)d.iPr;
+        }
+        // rows: rho, m_x, m_y, m_z, Theta
+        for (int row = 0; row < 5; row++) {
+            R f0, f1, f2, g0, g1, g2;
+            if (row == 0) { f0 = A.m[0]; f1 = A.m[1]; f2 = A.m[2]; }
+            else if (row < 4) {
+                const int r = row - 1;
+                f0 = r == 0 ? A.m[r] * u[0] + A.pp : A.m[r] * u[0];
+                f1 = r == 1 ? A.m[r] * u[1] + A.pp : A.m[r] * u[1];
+                f2 = r == 2 ? A.m[r] * u[2] + A.pp : A.m[r] * u[2];
+            } else {
+                f0 = A.m[0] * T0 + A.m[0] * A.thp;
+                f1 = A.m[1] * T0 + A.m[1] * A.thp;
+                f2 = A.m[2] * T0 + A.m[2] * A.thp;
+            }
+            if constexpr (VISC) {
+                if (row >= 1 && row <= 3) {
+                    const int r3 = 3 * (row - 1);
+                    f0 = f0 - mu * gown[r3]; f1 = f1 - mu * gown[r3 + 1]; f2 = f2 - mu * gown[r3 + 2];
+                } else if (row == 4) {
+                    f0 = f0 - imu * gown[9]; f1 = f1 - imu * gown[10]; f2 = f2 - imu * gown[11];
+                }
+            }
+            contravariant(J, f0, f1, f2, g0, g1, g2);
+            G[(row * 3 + 0) * NP + q] = g0;
+            if constexpr (YL) G[(row * 3 + 1) * NP + q] = g1;
+            G[(row * 3 + 2) * NP + q] = g2;
+        }
+    }
+    __syncthreads();
+
+    R res[5];  // volume - surface (= -r of the reference), over cV when AFF
+    {
+        const R* D0 = Dl;
+        const R* D1 = Dl + NX * NX;
+        const R* D2 = D1 + NY * NY;
+        for (int row = 0; row < 5; row++) {
+            const R* G0 = G + (row * 3 + 0) * NP;
+            const R* G1 = G + (row * 3 + 1) * NP;
+            const R* G2 = G + (row * 3 + 2) * NP;
+            // a sum per line: shorter chains, and less rounded off than in one
+            R v0 = 0, v1 = 0, v2 = 0;
+            for (int t = 0; t < NX; t++) v0 += D0[t * NX + i] * G0[t * NY * NZ + j * NZ + k];
+            if constexpr (YL)
+                for (int t = 0; t < NY; t++) v1 += D1[t * NY + j] * G1[i * NY * NZ + t * NZ + k];
+            for (int t = 0; t < NZ; t++) v2 += D2[t * NZ + k] * G2[i * NY * NZ + j * NZ + t];
+            res[row] = YL ? (v0 + v1) + v2 : v0 + v2;
+        }
+        for (int v = 0; v < 5; v++) keep_here(res[v]);
+    }
+#pragma unroll
+    for (int p = 0; p < PF; p++)
+        if (wave0 + p * threads < tasks) normal(tid + p * threads, ft[p]);
+    __syncthreads();
+    {
+        const R tr[kTraceRows] = {A.rp, A.m[0], A.m[1], A.m[2], A.tp, A.ir, A.thp, A.pp, rref, pref};
+        for (int r = 0; r < kTraceRows; r++) G[r * NPP + rk_prim_slot(q)] = tr[r];
+    }
+    __syncthreads();
+
+    auto face = [&](int t, const FaceTask<R>& F) {
+        int lt, tl;
+        task_of(t, lt, tl);
+        R* FL = LDS + lt * per_elem + kTraceRows * NPP + tl;   // face fluxes [5][NFN]
+        R flux[5] = {R(0), R(0), R(0), R(0), R(0)};
+        if (((F.meta >> 4) & 1) && !(MORT && ((F.meta >> 6) & 1))) {
+            const bool ghost = (F.meta >> 5) & 1;
+            const R* en = F.en;
+            int g, fa, fb, fnode;   // (again: not kept over the volume term)
+            locate_face_task<YF>(tl, NX, NY, NZ, g, fa, fb, fnode);
+            Trace<R> B, L, Q;
+            const R* Pf = LDS + lt * per_elem + rk_prim_slot(fnode);
+            B.rp = Pf[0 * NPP];
+            for (int c = 0; c < 3; c++) B.m[c] = Pf[(1 + c) * NPP];
+            B.tp = Pf[4 * NPP];
+            B.ir = Pf[5 * NPP];
+            B.thp = Pf[6 * NPP];
+            B.pp = Pf[7 * NPP];
+            const R rrefF = Pf[8 * NPP], prefF = Pf[9 * NPP];
+            const R mnB = B.m[0] * en[0] + B.m[1] * en[1] + B.m[2] * en[2];
+            R unQ, mnQ, mnL = mnB, unL = mnB * B.ir;
+            if (!ghost) {
+                Q.rp = F.rp;
+                for (int c = 0; c < 3; c++) Q.m[c] = F.m[c];
+                Q.tp = F.tp;
+                complete(Q, rrefF, prefF, T0, gam, d);
+                B.cu = speed_plus_c(B.m, B.ir, B.thp, T0, gR);
+                Q.cu = speed_plus_c(Q.m, Q.ir, Q.thp, T0, gR);
+                mnQ = Q.m[0] * en[0] + Q.m[1] * en[1] + Q.m[2] * en[2];
+                unQ = mnQ * Q.ir;
+                L = B;
+            } else {
+                const BcTable& bt = *d.bc;
+                const int pi = F.meta >> 8;
+                const double uv[3] = {bt.value[1][pi], bt.value[2][pi], bt.value[3][pi]};
+                ghost_trace(B, en, bt.kind[1][pi], uv, rrefF, T0, gR, Q, unQ);
+                mnQ = Q.m[0] * en[0] + Q.m[1] * en[1] + Q.m[2] * en[2];
+                L = Q;
+                mnL = mnQ;
+                unL = unQ;
+            }
+            rusanov_out(B, L, Q, mnB, mnL, mnQ, unL, unQ, en, T0, flux);
+            if constexpr (VISC) {
+                // central average of -mu grad . n; a boundary face takes the
+                // ghost gradient and the own density
+                const uint64_t na = (uint64_t)(ONE ? e0 : min(e0 + lt, d.nelem - 1)) * NP + fnode;
+                R gA[12], gB[12];
+                for (int c = 0; c < 12; c++) gA[c] = ldn<O32>(grd + (size_t)c * nb, na);
+                const R muA = (rrefF + B.rp) * (R)d.visc;
+                R vA[4], vB[4];
+                viscous_normal(gA, muA, (R)d.iPr, en, vA);
+                if (!ghost) {
+                    for (int c = 0; c < 12; c++) gB[c] = ldn<O32>(grd + (size_t)c * nb, F.node);
+                    viscous_normal(gB, (rrefF + F.rp) * (R)d.visc, (R)d.iPr, en, vB);
+                } else {
+                    ghost_gradient_r(*d.bc, (int)(F.meta >> 8), gA, gB);
+                    viscous_normal(gB, muA, (R)d.iPr, en, vB);
+                    for (int r = 0; r < 4; r++) vA[r] = vB[r];
+                }
+                for (int r = 0; r < 4; r++) flux[1 + r] = flux[1 + r] - (vA[r] + vB[r]) * R(0.5);
+            }
+            for (int v = 0; v < 5; v++) flux[v] = flux[v] * F.s;
+        }
+        for (int v = 0; v < 5; v++) FL[v * NFN] = flux[v];
+    };
+#pragma unroll
+    for (int p = 0; p < PF; p++)
+        if (wave0 + p * threads < tasks) face(tid + p * threads, ft[p]);
+    // (a compile-time shape whose tasks the passes above cover has no more)
+    if constexpr (!NPc || rk_face_nodes<YF>(NXc, NYc, NZc) > PF * NPc)
+        for (int t = tid + PF * threads; t < tasks; t += threads) {
+            prepare(t, entry(t), ft[0]);
+            normal(t, ft[0]);
+            face(t, ft[0]);
+        }
+    __syncthreads();
+    if (!active) return;
+
+    const R* FL = G + kTraceRows * NPP;
+    for (int g = 0; g < 6; g++) {
+        if (!YF && (g == 2 || g == 3)) continue;
+        if (!on_face(g, i, j, k, NX, NY, NZ)) continue;
+        int fa, fb;
+        face_ab(g, i, j, k, fa, fb);
+        if constexpr (MORT) {
+            const uint32_t meta = d.eface[(size_t)e * 6 + g].meta;
+            if ((meta >> 6) & 1) {
+                // 2:1 mortar side: its surface term, sign included, from the
+                // stage's mortar pre-pass
+                const size_t mi = ((size_t)(meta >> 8) * d.npfm + fa * (g < 2 ? NY : NZ) + fb) * 5;
+                R w = 1;
+                if constexpr (AFF) w = r_rcp((R)(d.emet[(size_t)e * 10 + 9] * d.wnode[q]));
+                for (int v = 0; v < 5; v++) {
+                    R x = (R)d.msurf[mi + v];
+                    if constexpr (is_dual<R>::value) x.d[0] = d.msurf_t[mi + v];
+                    res[v] += x * w;
+                }
+                continue;
+            }
+        }
+        int t = face_task_index(g, fa, fb, NX, NY, NZ);
+        if (!YF && g > 3) t -= 2 * NX * NZ;
+        // 1 / w_end of the face's direction (an integer but for one node)
+        const int n1 = g < 2 ? NZ : g < 4 ? NY : NX;
+        const R c = AFF ? R(n1 > 1 ? n1 * (n1 - 1) * 0.5f : 0.5f) : R(1);
+        for (int v = 0; v < 5; v++) res[v] -= FL[v * NFN + t] * c;
+    }
+    // L(q) = (volume - surface)/cV + buoyancy; increments and base
+    if constexpr (!AFF) {
+        const R icv = r_rcp(cvn);
+        for (int v = 0; v < 5; v++) res[v] = res[v] * icv;
+    }
+    if (d.buoyancy)
+        for (int c = 0; c < 3; c++) res[1 + c] += A.rp * (R)d.g[c];
+    for (int v = 0; v < 5; v++) {
+        const double out = pre[v] + a.bdt * value_of(res[v]);
+        if (a.last) stn<O32>(a.qout[v], n, out);
+        else stn<O32>(a.dout[v], n, (S)out);
+        if constexpr (is_dual<R>::value) {
+            const double tout = tpre[v] + a.bdt * res[v].d[0];
+            if (a.last) stn<O32>(a.tqout[v], n, tout);
+            else stn<O32>(a.tdout[v], n, tout);
+        }
+    }
+    if (a.check) {
+        bool bad = false;
+        for (int v = 0; v < 5; v++) bad |= !isfinite(value_of(res[v]));
+        if (bad) *a.flag = 1;
+    }
+}
+
+template <typename R, typename S, int X, int Y, int Z, bool DIN, bool AFF, bool VISC, bool MORT, bool YF>
+__global__ void __launch_bounds__(512) rk_stage_kernel(DgDev d, RkArgs<S> a) {
+    rk_stage_body<R, S, X, Y, Z, false, DIN, AFF, VISC, MORT, YF>(d, a);
+}
+
+// Compile-time element shape (X x Y x Z nodes), node offsets in 32 bits,
+// registers capped at W waves per SIMD: the most at which the shape does not
+// spill.  FP32 takes 76-80 registers and six waves (three work-groups per CU
+// at N = 7); FP64 114-126 and four, the shapes of several elements per
+// work-group (face tasks in two passes) up to 126 with an element index per
+// lane and three; a 2D group is one or two waves whose latency counts, and
+// measured faster with registers to spare (5 x 1 x 5 FP64: 21.2 us a step of
+// 62,500 nodes at two, 23.3 at three).  The viscous variant's extra gradient
+// state takes two less.
+template <typename R, int X, int Y, int Z, bool VISC>
+constexpr int rk_waves_per_simd() {
+    constexpr int np = X * Y * Z;
+    if constexpr (sizeof(R) == 4) return VISC ? 4 : 6;
+    return VISC || Y == 1 ? 2 : np > 128 ? 4 : 3;
+}
+
+template <typename R, typename S, int X, int Y, int Z, int W, bool DIN, bool AFF, bool VISC, bool MORT, bool YF>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(W)))
+rk_stage_kernel_fx(DgDev d, RkArgs<S> a) {
+    rk_stage_body<R, S, X, Y, Z, true, DIN, AFF, VISC, MORT, YF>(d, a);
+}
+
+template <typename R, typename S, int X, int Y, int Z, bool DIN, bool AFF, bool VISC, bool MORT, bool YF>
+static void launch_rk_kernel(const DgDev& d, const RkArgs<S>& a, unsigned blocks, int threads, size_t lds,
+                             hipStream_t st) {
+    constexpr int W = rk_waves_per_simd<R, X, Y, Z, VISC>();
+    if constexpr (X > 0 && !is_dual<R>::value) {
+        if (d.nb * sizeof(double) < (1ull << 32)) {
+            hipLaunchKernelGGL((rk_stage_kernel_fx<R, S, X, Y, Z, W, DIN, AFF, VISC, MORT, YF>), dim3(blocks),
+                               dim3(threads), lds, st, d, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((rk_stage_kernel<R, S, X, Y, Z, DIN, AFF, VISC, MORT, YF>), dim3(blocks), dim3(threads), lds,
+                       st, d, a);
+}
+
+template <typename R, typename S, int X, int Y, int Z, bool DIN, bool AFF>
+static void launch_rk_variant(const DgDev& d, const RkArgs<S>& a, unsigned blocks, int threads, size_t lds,
+                              hipStream_t st) {
+    // the tangent-linear instantiation has no viscous variant (the
+    // derivative entry points refuse diffusion)
+    const bool visc = !is_dual<R>::value && a.grad;
+    if constexpr (!is_dual<R>::value) {
+        if (visc) {
+            // 2:1 non-conforming meshes
+            if (d.nmort) launch_rk_kernel<R, S, X, Y, Z, DIN, AFF, true, true, true>(d, a, blocks, threads, lds, st);
+            else launch_rk_kernel<R, S, X, Y, Z, DIN, AFF, true, false, true>(d, a, blocks, threads, lds, st);
+            return;
+        }
+    }
+    if (d.nmort) {
+        launch_rk_kernel<R, S, X, Y, Z, DIN, AFF, false, true, true>(d, a, blocks, threads, lds, st);
+        return;
+    }
+    if constexpr (Y == 1) {
+        if (!d.yfaces) {
+            launch_rk_kernel<R, S, X, Y, Z, DIN, AFF, false, false, false>(d, a, blocks, threads, lds, st);
+            return;
+        }
+    }
+    launch_rk_kernel<R, S, X, Y, Z, DIN, AFF, false, false, true>(d, a, blocks, threads, lds, st);
+}
+
+template <typename R, typename S, int X, int Y, int Z>
+hipError_t launch_rk_t(const DgDev& d, const RkArgs<S>& a_in, hipStream_t st) {
+    RkArgs<S> a = a_in;
+    const int NP = d.np;
+    if (NP > 512) return hipErrorInvalidValue;
+    // elements per work-group: fill 256 threads, as far as the LDS allows;
+    // on a small mesh fewer, so that every CU gets about four work-groups
+    int epb = NP >= 256 ? 1 : 256 / NP;
+    while (epb > 1 && (rk_lds_bytes(d.npx, d.npy, d.npz, epb, sizeof(R)) > 65536 || d.nelem / epb < 1024)) epb--;
+    const int threads = (epb * NP + 63) / 64 * 64;
+    unsigned blocks = (d.nelem + epb - 1) / epb;
+    blocks = (blocks + 7) / 8 * 8;  // whole XCD chunks
+    const size_t lds = rk_lds_bytes(d.npx, d.npy, d.npz, epb, sizeof(R));
+    if (lds > 65536) return hipErrorInvalidValue;
+    if (X * Y * Z > 128 && epb != 1) return hipErrorInvalidValue;  // the body assumes one element
+    a.epb = epb;
+    // The per-element metric in FP64 (and its tangent) only: in FP32 its one
+    // rounding is the same for every element, and the error of rho' then grows
+    // with the steps (32 x 32 x 16 elements, N = 7, 200 steps: 7.9e-7 against
+    // 5.1e-7 with the per-node metric, whose roundings average out).
+    if constexpr (sizeof(R) != 4) {
+        if (d.affine) {
+            if (a.din[0]) launch_rk_variant<R, S, X, Y, Z, true, true>(d, a, blocks, threads, lds, st);
+            else launch_rk_variant<R, S, X, Y, Z, false, true>(d, a, blocks, threads, lds, st);
+            return hipGetLastError();
+        }
+    }
+    if (a.din[0]) launch_rk_variant<R, S, X, Y, Z, true, false>(d, a, blocks, threads, lds, st);
+    else launch_rk_variant<R, S, X, Y, Z, false, false>(d, a, blocks, threads, lds, st);
+    return hipGetLastError();
+}
+
+}  // namespace nsem
+
+// One element shape in every residual type.  Each shape is instantiated in a
+// translation unit of its own (dg_rk_shape_*.hip), so that they compile side
+// by side.
+#define NSEM_RK_SHAPE_(KIND, X, Y, Z)                                                                      \
+    KIND template hipError_t nsem::launch_rk_t<double, double, X, Y, Z>(const nsem::DgDev&,                \
+                                                                        const nsem::RkArgs<double>&, hipStream_t); \
+    KIND template hipError_t nsem::launch_rk_t<float, float, X, Y, Z>(const nsem::DgDev&,                  \
+                                                                      const nsem::RkArgs<float>&, hipStream_t); \
+    KIND template hipError_t nsem::launch_rk_t<nsem::Dual<1>, double, X, Y, Z>(                            \
+        const nsem::DgDev&, const nsem::RkArgs<double>&, hipStream_t);
+#define NSEM_RK_SHAPE(X, Y, Z) NSEM_RK_SHAPE_(, X, Y, Z)

@@ -133,6 +133,34 @@ def test_rk3_fp32_orders_against_fp64(oracle, tmp_path, case):
     dg2.close()
 
 
+# Edges of the stage kernel's dispatch: the compile-time 2D shapes of N = 5 and
+# 6, 2D decks whose y faces are walls (the variant with y-face tasks) beside
+# those without any, two elements per work-group with the last group half
+# empty (2197 elements), a viscous 2D shape.
+_CFG0 = [c for c in EULER_CASES if c["name"] == "cfg0_2d_n4"][0]
+_CFG0_VISC = [c for c in EULER_CASES if c["name"] == "cfg0_2d_visc"][0]
+_Y_WALLS = [p for p in _CFG0["patches"] if p[0] != "delete"]
+_Y_WALLS = _Y_WALLS[:-1] + [(_Y_WALLS[-1][0], _Y_WALLS[-1][1] + [(0, 1, 2, 3), (4, 5, 6, 7)])]
+STAGE_CASES = [dict(_CFG0, name="2d_n5", order=(5, 0, 5)), dict(_CFG0, name="2d_n6", order=(6, 0, 6)),
+               dict(_CFG0, name="2d_n4_y_walls", patches=_Y_WALLS),
+               dict(_E3_N3, name="e3_n3_ragged", ndiv=(13, 13, 13)),
+               dict(_CFG0_VISC, name="2d_n5_visc", order=(5, 0, 5))]
+
+
+@pytest.mark.parametrize("case", STAGE_CASES, ids=[c["name"] for c in STAGE_CASES])
+def test_rk3_stage_dispatch_edges(oracle, tmp_path, case):
+    """FP64 against the oracle within check_rk3_against_oracle's bounds, then
+    FP32 against FP64 on the same deck within those of the orders above: the
+    FP32 residual's error of m and rho' is a few 6e-8 of the terms that make
+    it up, and that of Theta' about 6e-8 |m| theta dt / dx a step, 1e-12 of
+    Theta_ref here."""
+    print(f"[gpu] rk3 stage {case['name']}", flush=True)
+    mesh, om, prm, dg, state = setup(oracle, tmp_path, case)
+    check_rk3_against_oracle(oracle, om, prm, dg, mesh.info.nbcs_field, *state, 3)
+    dg.close()
+    test_rk3_fp32_orders_against_fp64(oracle, tmp_path / "fp32", case)
+
+
 def test_rk3_conserves_mass_on_device(oracle, tmp_path):
     case = [c for c in EULER_CASES if c["name"] == "e3_n3"][0]
     mesh, om, prm, dg, state = setup(oracle, tmp_path, case)
